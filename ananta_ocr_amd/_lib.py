@@ -24,6 +24,12 @@ SIGNATURES = {
                                _p, _l, _p]),
     "dash_block_max_score": (_i, [_p, _l, _l, _i, _p, _p, _l, _p, _l, _l, _i, _i, _i, _i, _i,
                                   _i, _i, _p, _l, _l, _p]),
+    "dash_block_max_fused_workspace_size": (_i, [_i, _i, _i, ctypes.POINTER(_l)]),
+    "dash_block_max_fused": (_i, [_p, _l, _l, _i, _p, _p, _l, _p, _l, _l, _i, _i, _i, _i, _i,
+                                  _i, _i, _p, _l, _l, _p, _p, _l, _p]),
+    "dash_block_max_backward_workspace_size": (_i, [_i, _i, _i, _i, ctypes.POINTER(_l)]),
+    "dash_block_max_backward": (_i, [_p, _l, _l, _i, _p, _l, _p, _l, _l, _i, _i, _i, _i, _i, _i,
+                                     _p, _p, _l, _l, _p, _p, _p, _l, _p]),
     "dash_router_qk_norm": (_i, [_p, _i, _l, _l, _i, _i, _p, _p, _f, _p, _p, _i, _l, _l, _p, _p,
                                  _p]),
     "dash_router_front": (_i, [_p, _l, _l, _i, _i, _i, _p, _p, _p, _p, _p, _f, _p, _p, _i, _l, _l,

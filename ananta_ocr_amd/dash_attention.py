@@ -423,7 +423,16 @@ class DashAttention(nn.Module):
     def _block_scores_train(self, iq, ik, position_ids, nblk):
         """Indexer scores (dash_attention.py:801-835): for query t and block c the max
         over the block's keys j with j <= pos_t - LW of clamp(iq_t . ik_j, +-1e4),
-        -1e9 where the block has no such key; chunks of q_chunk queries."""
+        -1e9 where the block has no such key.  Index dim 128 and blocks of 32 to 128 keys run
+        in the library, which never forms the [S, S] scores (a 27,300-token row of blocks of 32:
+        the forward and backward of these tensor ops took 29 ms); others by tensor ops."""
+        if ops.block_max_train_ok(iq, ik, self.block_size):
+            return ops.block_max_train(iq, ik, position_ids, self.block_size, self.local_window,
+                                       nblk, self._block_scores_ops)
+        return self._block_scores_ops(iq, ik, position_ids, nblk)
+
+    def _block_scores_ops(self, iq, ik, position_ids, nblk):
+        """_block_scores_train by tensor ops, in chunks of q_chunk queries."""
         B, S, d = ik.shape
         bs = self.block_size
         pad = nblk * bs - S

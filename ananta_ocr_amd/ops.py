@@ -152,14 +152,107 @@ def block_max_score(q, k, pos, seg, block_size, num_key_blocks, local_window, mo
     Sk = k.shape[1]
     pos = _i32(pos)
     seg = _i32(seg)
-    out = torch.empty(B, C, num_key_blocks, dtype=torch.float32, device=q.device)
     lw = block_size if local_window is None else max(1, int(local_window))
+    if C >= BLOCK_MAX_FUSED_ROWS and _block_max_fused_ok(d, block_size):
+        return _block_max_fused(q, k, pos, seg, block_size, num_key_blocks, lw, mode)[0]
+    out = torch.empty(B, C, num_key_blocks, dtype=torch.float32, device=q.device)
     st_ = lib.dash_block_max_score(_ptr(q), q.stride(0), q.stride(1), C, _ptr(pos), _ptr(seg),
                                    pos.stride(0), _ptr(k), k.stride(0), k.stride(1), Sk, B, d,
                                    block_size, lw, num_key_blocks, mode, _ptr(out),
                                    out.stride(0), out.stride(1), _stream())
     _lib.check(st_, "dash_block_max_score")
     return out
+
+
+# Fewest query rows per sequence for the matrix-core block-max kernel, which splits every key
+# into bf16 parts first and works on 128 rows at a time.  2,730 keys in blocks of 32: 128 rows
+# 22.8 us against 19.8 us row by row, 2,730 rows 25.5 against 96.4; 27,300 rows and keys 551
+# against 7,514 us.
+BLOCK_MAX_FUSED_ROWS = 256
+
+
+def _block_max_fused_ok(d, block_size):
+    return d == 128 and block_size in (32, 64, 96, 128)
+
+
+def _f4_rows(x):
+    """fp32 rows the float4 loads take: contiguous features, 16-byte aligned rows."""
+    if x.stride(-1) != 1 or any(s % 4 for s in x.stride()[:-1]) or x.data_ptr() % 16:
+        x = x.contiguous()
+    return x
+
+
+def _block_max_fused(q, k, pos, seg, block_size, nblk, lw, mode, want_arg=False):
+    """dash_block_max_fused: (scores [B,C,nblk] fp32, winning keys uint8 or None)."""
+    lib = _lib.load()
+    q, k = _f4_rows(q), _f4_rows(k)
+    B, C, d = q.shape
+    nbytes = ctypes.c_int64(0)
+    _lib.check(lib.dash_block_max_fused_workspace_size(B, block_size, nblk, nbytes), "workspace")
+    ws = torch.empty(max(nbytes.value, 16), dtype=torch.uint8, device=q.device)
+    out = torch.empty(B, C, nblk, dtype=torch.float32, device=q.device)
+    arg = torch.empty(B, C, nblk, dtype=torch.uint8, device=q.device) if want_arg else None
+    st_ = lib.dash_block_max_fused(
+        _ptr(q), q.stride(0), q.stride(1), C, _ptr(pos), _ptr(seg), pos.stride(0), _ptr(k),
+        k.stride(0), k.stride(1), k.shape[1], B, d, block_size, lw, nblk, mode, _ptr(out),
+        out.stride(0), out.stride(1), _ptr(arg), _ptr(ws), ws.numel(), _stream())
+    _lib.check(st_, "dash_block_max_fused")
+    return out, arg
+
+
+def block_max_train_ok(iq, ik, block_size):
+    """Whether block_max_train takes these index queries and keys."""
+    return (iq.is_cuda and iq.dtype == torch.float32 and ik.dtype == torch.float32
+            and iq.shape[0] > 0 and iq.shape[1] > 0
+            and _block_max_fused_ok(iq.shape[-1], block_size))
+
+
+class _BlockMaxFn(torch.autograd.Function):
+    """Training block-max scores (dash_attention.py:801-835) with gradients to the index
+    queries and keys."""
+
+    @staticmethod
+    def forward(ctx, iq, ik, pos, block_size, lw, nblk, differentiable):
+        z, arg = _block_max_fused(iq, ik, pos, None, block_size, nblk, lw, 2,
+                                  want_arg=any(ctx.needs_input_grad[:2]))
+        ctx.save_for_backward(iq, ik, pos, arg)
+        ctx.cfg = (block_size, lw, nblk, differentiable)
+        return z
+
+    @staticmethod
+    def backward(ctx, dz):
+        iq, ik, pos, arg = ctx.saved_tensors
+        block_size, lw, nblk, differentiable = ctx.cfg
+        if torch.is_grad_enabled():            # create_graph: by tensor ops
+            g = torch.autograd.grad(differentiable(iq, ik, pos, nblk), (iq, ik), dz,
+                                    create_graph=True)
+            return (*g, None, None, None, None, None)
+        lib = _lib.load()
+        q, k, dz = _f4_rows(iq), _f4_rows(ik), dz.float()
+        if dz.stride(-1) != 1:
+            dz = dz.contiguous()
+        B, C, d = q.shape
+        Sk = k.shape[1]
+        nbytes = ctypes.c_int64(0)
+        _lib.check(lib.dash_block_max_backward_workspace_size(B, C, Sk, nblk, nbytes), "workspace")
+        ws = torch.empty(max(nbytes.value, 16), dtype=torch.uint8, device=q.device)
+        dq = torch.empty(B, C, d, dtype=torch.float32, device=q.device)
+        dk = torch.empty(B, Sk, d, dtype=torch.float32, device=q.device)
+        st_ = lib.dash_block_max_backward(
+            _ptr(q), q.stride(0), q.stride(1), C, _ptr(pos), pos.stride(0), _ptr(k), k.stride(0),
+            k.stride(1), Sk, B, d, block_size, lw, nblk, _ptr(arg), _ptr(dz), dz.stride(0),
+            dz.stride(1), _ptr(dq), _ptr(dk), _ptr(ws), ws.numel(), _stream())
+        _lib.check(st_, "dash_block_max_backward")
+        return dq, dk, None, None, None, None, None
+
+
+def block_max_train(iq, ik, position_ids, block_size, local_window, nblk, differentiable):
+    """Training indexer scores z [B,S,nblk] fp32 of index queries / keys [B,S,128] fp32:
+    max over each block's keys j <= position - local_window of clamp(iq . ik_j, +-1e4),
+    -1e9 where there is none, with autograd to iq and ik.  differentiable(iq, ik,
+    position_ids, nblk): the same scores by tensor ops, for a graph of the gradient."""
+    pos = _i32(position_ids.expand(iq.shape[:2]))
+    return _BlockMaxFn.apply(iq, ik, pos, block_size, int(local_window), nblk, differentiable)
 
 
 def router_qk_norm(proj, wq, wk, eps, cos=None, sin=None):

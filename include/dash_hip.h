@@ -88,6 +88,37 @@ int dash_block_max_score(const float* q, int64_t q_sb, int64_t q_st, int C,
                          float* out, int64_t o_sb, int64_t o_sc, void* stream);
 
 /*
+ * The same scores on the matrix cores: d = 128, block_size 32, 64, 96 or 128, rows of q and
+ * k 16-byte aligned (strides multiples of 4); else unsupported.  mode 2 = the training form
+ * (mode 0, but a NaN score makes its block's score NaN).  arg [B, C, nblk] (or NULL): the
+ * winning key of every block, within the block, 255 where there is no single one; the
+ * backward call reads it.  ws: 16-byte aligned, of the size
+ * dash_block_max_fused_workspace_size gives; its contents need not be kept.
+ */
+int dash_block_max_fused_workspace_size(int B, int block_size, int nblk, int64_t* bytes);
+int dash_block_max_fused(const float* q, int64_t q_sb, int64_t q_st, int C,
+                         const int32_t* pos, const int32_t* seg, int64_t ps_sb,
+                         const float* k, int64_t k_sb, int64_t k_st, int Sk, int B,
+                         int d, int block_size, int local_window, int nblk, int mode,
+                         float* out, int64_t o_sb, int64_t o_sc, uint8_t* arg, void* ws,
+                         int64_t ws_bytes, void* stream);
+
+/*
+ * Gradients of mode 2 (no segment starts) for the gradient g[b*g_sb + t*g_sc + c] of its
+ * scores, which may be mostly zero: dq [B, C, 128] and dk [B, Sk, 128] fp32 contiguous.  The
+ * keys that attain a block's maximum share its gradient equally; a score beyond the clamp
+ * passes none.  nblk = ceil(Sk / block_size).
+ */
+int dash_block_max_backward_workspace_size(int B, int C, int Sk, int nblk, int64_t* bytes);
+int dash_block_max_backward(const float* q, int64_t q_sb, int64_t q_st, int C,
+                            const int32_t* pos, int64_t ps_sb, const float* k,
+                            int64_t k_sb, int64_t k_st, int Sk, int B, int d,
+                            int block_size, int local_window, int nblk,
+                            const uint8_t* arg, const float* g, int64_t g_sb,
+                            int64_t g_sc, float* dq, float* dk, void* ws,
+                            int64_t ws_bytes, void* stream);
+
+/*
  * Router front end after the index projections: Gemma RMSNorm (scale 1 + w, eps,
  * activations clamped to +-1e4), optional RoPE (rotate-half, cos/sin rows of the
  * first d dims) and the finiteness guards of _router_qk (modeling_deepseekv2.py:336-348)

@@ -1,0 +1,128 @@
+"""The matrix-core block-max scores (dash_block_max_fused) and their gradient
+(dash_block_max_backward) on the GPU against 64-bit tensor ops: tile and block edges, ragged
+lengths, packed positions, segment starts, equal keys (which share a gradient), scores at
+the clamp and operands that are not finite.
+
+Score tolerance: an fp32 dot product of 128 terms in any order is within 128 * 2^-24 of the
+sum of the terms' magnitudes."""
+
+import math
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from ananta_ocr_amd import ops
+from ananta_ocr_amd.dash_attention import DashAttention
+from oracle import dash_oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+DOT = 128 * 2.0 ** -24
+
+
+def _router(bs, lb):
+    sp = dict(sparse_block_size=bs, sparse_local_block=lb, sparse_index_dim=128)
+    return DashAttention(SimpleNamespace(num_attention_heads=2, hidden_size=256,
+                                         rms_norm_eps=1e-6, sparse_attention_config=sp)).to(DEV)
+
+
+def _magnitude(q, k, bs, nblk):
+    """[B, C, nblk] largest sum of |q_i k_i| of a block."""
+    m = q.abs() @ k.abs().transpose(1, 2)
+    return torch.nn.functional.pad(m, (0, nblk * bs - k.shape[1])).view(*m.shape[:2], nblk, bs).amax(-1)
+
+
+@pytest.mark.parametrize("B,S,bs,lb", [(1, 1, 32, 1), (2, 31, 32, 1), (1, 333, 32, 4),
+                                       (2, 700, 64, 2), (1, 385, 96, 1), (1, 641, 128, 1),
+                                       (1, 4200, 32, 4), (1, 5000, 64, 1)])
+def test_training_scores_and_gradients(B, S, bs, lb):
+    g = torch.Generator().manual_seed(S + bs)
+    r = _router(bs, lb)
+    nblk = (S + bs - 1) // bs
+    iq, ik = (torch.randn(B, S, 128, generator=g) for _ in range(2))
+    if S > 300:
+        ik[:, 40:44] = ik[:, 40:41]                 # equal keys within one block
+        ik[:, 70] = 0.0
+        iq[:, S - 1] *= 2.0e4                       # scores beyond the clamp
+        iq[0, S - 2] = 1.0e19                       # beyond the bf16 parts' range
+        ik[0, 100] *= 1.0e19
+    pos = torch.arange(S).expand(B, S).clone()
+    if B > 1:
+        pos[1] = torch.cat([torch.arange(S // 2), torch.arange(S - S // 2)])
+    iq, ik, pos = iq.to(DEV), ik.to(DEV), pos.to(DEV)
+    a, b = iq.clone().requires_grad_(), ik.clone().requires_grad_()
+    assert ops.block_max_train_ok(a, b, bs)
+    z = r._block_scores_train(a, b, pos, nblk)
+    c, d = iq.double().requires_grad_(), ik.double().requires_grad_()
+    ref = r._block_scores_train(c, d, pos, nblk)    # 64-bit inputs: the tensor ops
+    tol = DOT * _magnitude(iq.double(), ik.double(), bs, nblk)
+    assert torch.all((z.double() - ref).abs() <= tol.clamp(max=1e30) + 1e-30)
+    # a gradient on a few entries of each row, the masked ones included
+    dz = torch.randn(z.shape, generator=g).to(DEV)
+    dz = torch.where(torch.rand(z.shape, generator=g).to(DEV) < 0.3, dz, torch.zeros_like(dz))
+    z.backward(dz)
+    ref.backward(dz.double())
+    for x, y in ((a, c), (b, d)):
+        # sums of up to 0.3 S terms in fp32, in another order
+        bound = 1e-5 * y.grad.abs().amax(-1, keepdim=True) + 1e-5
+        assert torch.all((x.grad.double() - y.grad).abs() <= bound)
+    z2 = r._block_scores_train(a, b, pos, nblk)     # the same gradient bits on every run
+    again = torch.autograd.grad(z2, (a, b), dz)
+    assert torch.equal(again[0], a.grad) and torch.equal(again[1], b.grad)
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("B,C,Sk,bs,lw", [(2, 64, 64, 32, 32), (1, 300, 1111, 64, 100),
+                                          (2, 129, 500, 96, 1), (1, 200, 2500, 128, 128)])
+def test_scores_match_oracle(B, C, Sk, bs, lw, mode, monkeypatch):
+    monkeypatch.setattr(ops, "BLOCK_MAX_FUSED_ROWS", 1)
+    g = torch.Generator().manual_seed(C + bs + mode)
+    q, k = torch.randn(B, C, 128, generator=g), torch.randn(B, Sk, 128, generator=g)
+    pos = torch.randint(0, Sk, (B, C), generator=g)
+    nblk = (Sk + bs - 1) // bs + 1                  # one block past the keys
+    seg = (pos // 3) if mode == 1 else torch.zeros_like(pos)
+    out = ops.block_max_score(q.to(DEV), k.to(DEV), pos.to(DEV), seg.to(DEV), bs, nblk, lw,
+                              mode=mode).cpu()
+    if mode == 1:
+        ref = O.block_max_score(q.double().float(), k, pos, seg, bs, nblk, lw)
+    else:
+        ref = O.block_scores_indexer(q, k, pos, nblk, bs, lw)
+    seen = ref > -5e8
+    assert torch.equal(out[~seen], ref[~seen])
+    tol = 2 * DOT * _magnitude(q, k, bs, nblk)      # both sides are fp32
+    assert torch.all((out - ref).abs()[seen] <= tol[seen])
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_scores_of_values_that_are_not_finite(mode, monkeypatch):
+    """The matrix-core kernel gives what the row-by-row kernel gives."""
+    g = torch.Generator().manual_seed(3)
+    q, k = torch.randn(1, 96, 128, generator=g), torch.randn(1, 400, 128, generator=g)
+    q[0, 5, 3], q[0, 6, 4], k[0, 33, 7], k[0, 95, 0] = math.inf, math.nan, -math.inf, math.nan
+    k[0, 200:216] = 3.0e38
+    pos = torch.full((1, 96), 399)
+    args = (q.to(DEV), k.to(DEV), pos.to(DEV), None, 32, 13, 32)
+    old = ops.block_max_score(*args, mode=mode)
+    monkeypatch.setattr(ops, "BLOCK_MAX_FUSED_ROWS", 1)
+    out = ops.block_max_score(*args, mode=mode)
+    assert torch.equal(out.isnan(), old.isnan()) and torch.equal(out.isinf(), old.isinf())
+    fin = old.isfinite()
+    torch.testing.assert_close(out[fin], old[fin], atol=1e-4, rtol=1e-5)
+    assert torch.equal(out[~fin & ~old.isnan()], old[~fin & ~old.isnan()])
+
+
+def test_gradient_of_the_gradient():
+    """create_graph goes through the tensor ops."""
+    r = _router(32, 1)
+    a, b = (torch.randn(1, 100, 128, device=DEV, requires_grad=True) for _ in range(2))
+    pos = torch.arange(100, device=DEV)[None]
+    z = r._block_scores_train(a, b, pos, 4)
+    w = torch.randn_like(z)
+    (da,) = torch.autograd.grad(z, a, w, create_graph=True)
+    (db,) = torch.autograd.grad(da.square().sum(), b)
+    z2 = r._block_scores_ops(a, b, pos, 4)
+    (da2,) = torch.autograd.grad(z2, a, w, create_graph=True)
+    (db2,) = torch.autograd.grad(da2.square().sum(), b)
+    torch.testing.assert_close(da, da2, atol=1e-5, rtol=1e-5)
+    torch.testing.assert_close(db, db2, atol=1e-4, rtol=1e-4)
