@@ -109,6 +109,12 @@ struct PrefillArgs {
   int split_parts;                     // parts per (sequence, head): the sum over tiles
   bf16* split_o;                       // [tiles, kSplitMax, kPfTQ, D] bf16, dims in order
   float* split_lse;                    // [tiles, kSplitMax, kPfTQ]
+  // extend (null otherwise): query row t of sequence b is at position ctx[b] + t of a
+  // cached sequence of klen[b] keys (at most key_cap); S, cu and the tiles count query
+  // rows, blocks count keys
+  const int32_t* ctx;                  // [B]
+  const int32_t* klen;                 // [B]
+  int key_cap;
 };
 
 // Upper bound of the items of tile t (no plan) of a sequence of S tokens: its
@@ -132,6 +138,13 @@ __host__ __device__ inline int tile_parts(int t, int S, int lw, int bs, int K, i
 
 __device__ __forceinline__ int seq_len(const PrefillArgs& a, int b) {
   return a.cu ? a.cu[b + 1] - a.cu[b] : a.S;
+}
+// Keys of sequence b, and the position of its query row t among them.
+__device__ __forceinline__ int key_len(const PrefillArgs& a, int b) {
+  return a.klen ? min(max(a.klen[b], 0), a.key_cap) : seq_len(a, b);
+}
+__device__ __forceinline__ int q_pos_of(const PrefillArgs& a, int b, int t, int klen) {
+  return a.ctx ? min(a.ctx[b] + t, klen - 1) : t;
 }
 __device__ __forceinline__ int64_t row0(const PrefillArgs& a, int b) {
   return a.cu ? (int64_t)a.cu[b] : (int64_t)b * a.S;
@@ -235,7 +248,8 @@ __global__ __launch_bounds__(kPfTQ) void prefill_plan_kernel(PrefillArgs a) {
   const int len = seq_len(a, b);
   const int t0 = blockIdx.x * kPfTQ;
   if (t0 >= len) return;
-  const int nblk = (len + a.bs - 1) / a.bs;
+  const int klen = key_len(a, b);
+  const int nblk = (klen + a.bs - 1) / a.bs;
   for (int i = tid; i < nblk; i += kPfTQ) sCnt[i] = 0;
   __syncthreads();
   const int t = t0 + tid;
@@ -243,7 +257,7 @@ __global__ __launch_bounds__(kPfTQ) void prefill_plan_kernel(PrefillArgs a) {
   uint64_t keep_all = 0;
   if (t < len) {
     const int km = a.kmin ? a.kmin[row] : 0;
-    const int ls = t - a.lw + 1;
+    const int ls = q_pos_of(a, b, t, klen) - a.lw + 1;
     for (int g0 = 0; g0 < a.K; g0 += kPfMaxK) {
       int32_t c[kPfMaxK];
       uint32_t vmask, keep_mask = 0;
@@ -330,7 +344,8 @@ __global__ __launch_bounds__(1024) void prefill_scan_kernel(PrefillArgs a) {
   __shared__ int32_t sWave[2][16];
   const int b = blockIdx.x, tid = threadIdx.x, lane = wave_lane(), wv = tid / kWave;
   const int len = seq_len(a, b);
-  const int nblk = len > 0 ? (len + a.bs - 1) / a.bs : 0;
+  const int klen = key_len(a, b);
+  const int nblk = klen > 0 ? (klen + a.bs - 1) / a.bs : 0;
   int32_t* cnt = a.blk_count + (int64_t)b * a.nblk_cap;
   // two entries per thread
   int v0 = 0, v1 = 0;
@@ -440,7 +455,7 @@ __global__ __launch_bounds__(kPfTQ) void prefill_scatter_kernel(PrefillArgs a) {
   const int len = seq_len(a, b);
   const int t0 = blockIdx.x * kPfTQ;
   if (t0 >= len) return;
-  const int nblk = (len + a.bs - 1) / a.bs;
+  const int nblk = (key_len(a, b) + a.bs - 1) / a.bs;
   for (int i = tid; i < nblk; i += kPfTQ) sFill[i] = 0;
   __syncthreads();
   const int t = t0 + tid;
@@ -488,10 +503,11 @@ __global__ __launch_bounds__(kPfTQ) void prefill_scatter_kernel(PrefillArgs a) {
         int64_t rc, pp;
         if (scatter_target(a.chunk_cap, a.ppos, pos0, ch[s], q, &rc, &pp)) {
           rec[rc * kRec + kRecHead + q % kPfCH] = (int32_t)(slot - base);
-          a.spos[slot] = (int32_t)pp;
+          if (a.spos) a.spos[slot] = (int32_t)pp;
         } else {                                       // never with consistent counts
           atomicOr(a.err, 2);
-          a.spos[slot] = -1;                           // the tile kernel skips the slot
+          if (a.spos) a.spos[slot] = -1;               // the tile kernel skips the slot
+          else a.kind[slot] = 0;                       // the extend's merge skips it
         }
       }
   }
@@ -1709,6 +1725,7 @@ inline PlanLayout plan_layout(int B, int H, int S_max, int64_t rows, int K, int 
 }  // namespace dash
 
 #include "dash_prefill_bwd.h"
+#include "dash_extend.h"
 
 namespace dash {
 // Workspace of the backward: the plan (as the forward's, every routed pair

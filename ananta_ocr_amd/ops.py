@@ -806,6 +806,50 @@ def attn_rows(q, k, v, idx, bias, valid, q_pos, row_seq, block_size, local_windo
     return out
 
 
+# Fewest query rows of an extend step for the block-grouped matrix-core path.  Up to 128 rows
+# both paths take the step's launch time (window 512, 16 blocks of 64, caches of 13,650 tokens:
+# 345 us row by row, 347 grouped); 256 rows 484 against 347, 2,048 rows 2,849 against 368.
+EXTEND_ROWS = 128
+
+
+def attn_extend_ok(q, k, v, K, block_size, page_size, num_blocks, scale):
+    """Whether attn_extend takes these rows (else attn_rows)."""
+    return (q.shape[0] >= EXTEND_ROWS and q.shape[2] == 128 and block_size in (32, 64)
+            and page_size == block_size and K <= 64 and num_blocks <= 2048 and scale > 0
+            and q.shape[0] * q.shape[1] * max(K, 1) < 2 ** 31)
+
+
+def attn_extend(q, k, v, idx, bias, valid, seq_lens, context_lens, cu_seqlens_q, max_query_len,
+                block_table, block_size, local_window, scale, out_dtype=torch.float32):
+    """attn_rows for the rows of an extend step: row cu_seqlens_q[b] + i is position
+    context_lens[b] + i of request b (dash_attn_extend: pairs grouped by key block, on the
+    matrix cores).  q [T,H,128], k/v pages [pages, block_size, H, 128], idx/bias/valid [T,K],
+    lengths and tables int32.  Returns out [T,H,128] (out_dtype)."""
+    _need_gpu(q, k, v, idx, bias, valid)
+    lib = _lib.load()
+    T, H, D = q.shape
+    qr, k, v = (_rows(x.to(torch.bfloat16)) for x in (q, k, v))
+    bt, lens, ctx, cu = (_i32(x) for x in (block_table, seq_lens, context_lens, cu_seqlens_q))
+    B, P = bt.shape
+    K = idx.shape[-1]
+    idx_c, valid_c = _i32(idx.reshape(T, K)), _u8(valid.reshape(T, K))
+    bias_c = bias.reshape(T, K).float().contiguous()
+    nbytes = ctypes.c_int64(0)
+    _lib.check(lib.dash_attn_extend_workspace_size(B, H, int(max_query_len), T, K, P, nbytes),
+               "workspace")
+    ws = torch.empty(nbytes.value, dtype=torch.uint8, device=q.device)
+    out = torch.empty(T, H, D, dtype=out_dtype, device=q.device)
+    st_ = lib.dash_attn_extend(
+        _ptr(qr), qr.stride(0), qr.stride(1), _ptr(k), k.stride(2), k.stride(1), k.stride(0),
+        _ptr(v), v.stride(2), v.stride(1), v.stride(0), _ptr(bt), bt.stride(0), _ptr(lens),
+        _ptr(ctx), _ptr(cu), _ptr(idx_c), _ptr(valid_c), _ptr(bias_c), K, _ptr(out),
+        int(out_dtype == torch.bfloat16), out.stride(0), out.stride(1), B, H, T,
+        int(max_query_len), P, D, int(block_size), int(local_window), float(scale), _ptr(ws),
+        ws.numel(), _stream())
+    _lib.check(st_, "dash_attn_extend")
+    return out
+
+
 def attn_decode_rows(q, k, v, idx, bias, valid, q_pos, block_size, local_window, scale,
                      seq_lens=None, block_table=None, page_size=None, out_dtype=torch.float32):
     """Decode attention for Lq query rows per sequence, each at its own position.

@@ -144,6 +144,7 @@ def extend_prefill(state, q, k_cache, v_cache, idx_q, idx_k, head_cls, block_siz
     ctx = context_lens.to(device=dev, dtype=torch.int64)
     cu = cu_seqlens_q.to(device=dev, dtype=torch.int64)
     state.refresh_from(idx_k, head_cls, block_size, block_table, seq, ctx // block_size)
+    max_query_len = ops._max_len(cu, max_query_len)
     P = block_table.shape[1]
     pages = block_table.to(torch.int64).clamp(0, state.kbar.shape[0] - 1)
     kb_seq = state.kbar.index_select(0, pages.reshape(-1)).view(B, P, -1)
@@ -158,9 +159,14 @@ def extend_prefill(state, q, k_cache, v_cache, idx_q, idx_k, head_cls, block_siz
     width = max(1, min(int(K), int(topm))) if int(topm) > 0 else max(1, int(K))
     idx, bias, valid = ops.route(z, block_cand, idx_scale, floor, sigma, K, topm,
                                  row_nblk=nblk_b.index_select(0, row_seq), width=width)
-    out = ops.attn_rows(q, k_cache, v_cache, idx, bias, valid, q_pos, row_seq, block_size,
-                        local_blocks * block_size, scale, seq_lens=seq, block_table=block_table,
-                        page_size=block_size, out_dtype=out_dtype)
+    if ops.attn_extend_ok(q, k_cache, v_cache, idx.shape[-1], block_size, block_size, P, scale):
+        out = ops.attn_extend(q, k_cache, v_cache, idx, bias, valid, seq, ctx, cu, max_query_len,
+                              block_table, block_size, local_blocks * block_size, scale,
+                              out_dtype=out_dtype)
+    else:
+        out = ops.attn_rows(q, k_cache, v_cache, idx, bias, valid, q_pos, row_seq, block_size,
+                            local_blocks * block_size, scale, seq_lens=seq,
+                            block_table=block_table, page_size=block_size, out_dtype=out_dtype)
     if return_routing:
         return out, (idx, bias, valid.bool()), q_pos
     return out

@@ -367,6 +367,31 @@ int dash_attn_decode(const void* q, int64_t q_sb, int64_t q_sh,
                      float scale, int nsplit, void* workspace, int64_t workspace_bytes,
                      void* stream);
 
+/* Workspace bytes dash_attn_extend needs. */
+int dash_attn_extend_workspace_size(int B, int H, int max_query_len, int64_t T, int K, int nblk,
+                                    int64_t* bytes);
+
+/*
+ * Attention of an extend step over a paged cache (unlimited_ocr_v2_backend.py:1302-1335):
+ * the query rows cu_seqlens_q[b] .. cu_seqlens_q[b + 1] - 1 of q [T, H, 128] are positions
+ * context_lens[b] + i of request b, whose cache holds seq_lens[b] keys in pages of
+ * block_size tokens (pages block_table[b][c], c < nblk; element (page, token, head) at
+ * page * sp + token * st + head * sh).  Each row attends its window and the keys below the
+ * window of its routed blocks idx / valid / bias [T, K], as a query of dash_attn_decode
+ * with fp32 scores, weights and sums; a row's result does not depend on the other rows.
+ * block_size 32 or 64, K <= 64, nblk <= 2048, scale > 0.
+ */
+int dash_attn_extend(const void* q, int64_t q_st, int64_t q_sh,
+                     const void* k, int64_t k_sh, int64_t k_st, int64_t k_sp,
+                     const void* v, int64_t v_sh, int64_t v_st, int64_t v_sp,
+                     const int32_t* block_table, int64_t table_stride, const int32_t* seq_lens,
+                     const int32_t* context_lens, const int32_t* cu_seqlens_q,
+                     const int32_t* idx, const uint8_t* valid, const float* bias, int K,
+                     void* out, int out_bf16, int64_t o_st, int64_t o_sh,
+                     int B, int H, int64_t T, int max_query_len, int nblk, int D,
+                     int block_size, int local_window, float scale,
+                     void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Workspace bytes dash_decode_step needs (the window and routed partials and the
  * routing words the routers hand to the same launch). */
 int dash_decode_step_workspace_size(int B, int H, int D, int block_size, int local_window,

@@ -1,0 +1,123 @@
+"""The block-grouped extend attention (ops.attn_extend) against the row-by-row decode kernels
+(ops.attn_rows) and 64-bit arithmetic.
+
+Both hold scores, weights and sums in 32 bits.  A sum of n products of magnitude at most w in
+another order differs by at most n 2^-24 w; with the weights normalised and n <= 2,500 keys
+that is 1.5e-4 of the largest |v|, and in the usual square-root growth 3e-6; 2e-5 is stated.
+"""
+
+import math
+
+import pytest
+import torch
+
+from ananta_ocr_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _make(ctxs, news, H, bs, K, seed, lw, pad=0):
+    g = torch.Generator().manual_seed(seed)
+    lens = [a + b for a, b in zip(ctxs, news)]
+    P = max((n + bs - 1) // bs for n in lens) + pad
+    pool = sum((n + bs - 1) // bs for n in lens) + 2
+    perm = torch.randperm(pool, generator=g)
+    table = torch.full((len(lens), P), 10 ** 8, dtype=torch.int32)   # unused entries: no page
+    k = (torch.randn(pool, bs, H, 128, generator=g) * 0.7).bfloat16()
+    v = torch.randn(pool, bs, H, 128, generator=g).bfloat16()
+    o = 0
+    for b, n in enumerate(lens):
+        c = (n + bs - 1) // bs
+        table[b, :c] = perm[o:o + c].to(torch.int32)
+        if n % bs:                                   # rows past the end are never read
+            v[perm[o + c - 1], n % bs:] = float("nan")
+            k[perm[o + c - 1], n % bs:] = float("nan")
+        o += c
+    T = sum(news)
+    q = (torch.randn(T, H, 128, generator=g) * 0.7).bfloat16()
+    # block ids in and out of range, repeated, within the window, and not valid
+    idx = torch.randint(-1, P + 2, (T, K), generator=g, dtype=torch.int32)
+    bias = torch.randn(T, K, generator=g)
+    valid = torch.rand(T, K, generator=g) < 0.8
+    cu = torch.tensor([0] + news).cumsum(0).to(torch.int32)
+    return q, k, v, idx, bias, valid, lens, table, cu
+
+
+def _exact(q, k, v, idx, bias, valid, lens, table, cu, ctxs, bs, lw, scale, rows):
+    out = torch.zeros(len(rows), q.shape[1], 128, dtype=torch.float64)
+    for i, r in enumerate(rows):
+        b = int((cu[1:] <= r).sum())
+        qp = min(ctxs[b] + r - int(cu[b]), lens[b] - 1)
+        n = (lens[b] + bs - 1) // bs
+        pg = table[b, :n].long()
+        kk = k[pg].flatten(0, 1)[:lens[b]].double()
+        vv = v[pg].flatten(0, 1)[:lens[b]].double()
+        ls = qp - lw + 1
+        add = torch.full((lens[b],), -math.inf, dtype=torch.float64)
+        add[max(ls, 0):qp + 1] = 0.0
+        seen = set()
+        for s in range(idx.shape[1]):
+            c = int(idx[r, s])
+            if not valid[r, s] or c < 0 or c >= n or c * bs >= ls or c in seen:
+                continue
+            seen.add(c)
+            add[c * bs:min((c + 1) * bs, ls, lens[b])] = float(bias[r, s])
+        w = torch.softmax(torch.einsum("hd,nhd->hn", q[r].double(), kk) * scale + add, -1)
+        out[i] = torch.einsum("hn,nhd->hd", w, vv)
+    return out
+
+
+@pytest.mark.parametrize("ctxs,news,H,bs,lw,K", [
+    ([0], [128], 2, 64, 128, 8),              # whole tiles from the first token
+    ([63, 0, 700], [1, 129, 127], 3, 64, 256, 16),
+    ([1, 31, 32], [31, 33, 96], 2, 32, 128, 12),
+    ([2000], [65], 2, 32, 96, 64),            # four groups of slots
+    ([500, 90], [64, 300], 1, 64, 512, 5),    # slots not in fours; rows without routed keys
+    ([1234], [700], 4, 64, 512, 1),           # chunks of more than 256 pairs
+    ([17, 3000], [40, 30], 10, 64, 1000, 17),  # window not a multiple of the item
+])
+def test_extend_attention_matches_rows_and_exact(ctxs, news, H, bs, lw, K):
+    data = _make(ctxs, news, H, bs, K, sum(news) + K, lw, pad=1)
+    q, k, v, idx, bias, valid, lens, table, cu = data
+    scale = 1.0 / math.sqrt(128)
+    T = q.shape[0]
+    d = [x.to(DEV) for x in (q, k, v, idx, bias, valid)]
+    ctx = torch.tensor(ctxs, dtype=torch.int32, device=DEV)
+    ln = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    seq = torch.arange(len(news)).repeat_interleave(torch.tensor(news)).to(DEV)
+    pos = ctx[seq] + torch.arange(T, device=DEV) - cu.to(DEV)[seq]
+    got = ops.attn_extend(*d, ln, ctx, cu.to(DEV), max(news), table.to(DEV), bs, lw, scale)
+    # the row path reads table entries of used pages only, too
+    old = ops.attn_rows(*d, pos, seq, bs, lw, scale, seq_lens=ln, block_table=table.to(DEV),
+                        page_size=bs)
+    assert (got - old).abs().max().item() <= 2e-5 * old.abs().max().item()
+    rows = sorted(set(torch.linspace(0, T - 1, 40).long().tolist()))
+    ref = _exact(*data, ctxs, bs, lw, scale, rows)
+    err = (got[rows].cpu().double() - ref).norm() / ref.norm()
+    old_err = (old[rows].cpu().double() - ref).norm() / ref.norm()
+    assert err <= 2 * old_err + 2e-7, (err, old_err)
+    half = ops.attn_extend(*d, ln, ctx, cu.to(DEV), max(news), table.to(DEV), bs, lw, scale,
+                           out_dtype=torch.bfloat16)
+    assert torch.equal(half, got.bfloat16())
+
+
+def test_extend_attention_rows_do_not_depend_on_each_other():
+    """Rows in another batch (other tiles, chunks and requests beside them), and q, k and v
+    with other strides: the same bits."""
+    ctxs, news, H, bs, lw, K = [300, 900], [200, 333], 2, 64, 256, 8
+    q, k, v, idx, bias, valid, lens, table, cu = _make(ctxs, news, H, bs, K, 3, lw)
+    scale = 0.1
+    both = ops.attn_extend(*[x.to(DEV) for x in (q, k, v, idx, bias, valid)],
+                           torch.tensor(lens, device=DEV), torch.tensor(ctxs, device=DEV),
+                           cu.to(DEV), max(news), table.to(DEV), bs, lw, scale)
+    cut = 100                                  # request 1 from its 100th new row on
+    r = slice(news[0] + cut, sum(news))
+    qs = torch.stack([q[r], q[r]], 1).to(DEV)[:, 1]                 # strided rows
+    ks, vs = (torch.cat([x, x], 2).to(DEV)[:, :, H:] for x in (k, v))
+    one = ops.attn_extend(qs, ks, vs, *[x[r].to(DEV) for x in (idx, bias, valid)],
+                          torch.tensor(lens[1:], device=DEV),
+                          torch.tensor([ctxs[1] + cut], device=DEV),
+                          torch.tensor([0, news[1] - cut], device=DEV), news[1] - cut,
+                          table[1:].to(DEV), bs, lw, scale)
+    assert torch.equal(one, both[r])
