@@ -559,7 +559,7 @@ extern "C" int dash_attn_extend(
   const int nclear = (int)((L.clear_end - L.count) / 4);
   hipLaunchKernelGGL(prefill_clear_kernel, dim3((nclear + 255) / 256), dim3(256), 0, st, p.blk_count,
                      nclear);
-  if (K > 0) hipLaunchKernelGGL(prefill_plan_kernel, dim3(L.ntiles_cap, B), dim3(kPfTQ), 0, st, p);
+  if (K > 0) launch_plan(p, L.ntiles_cap, st);
   hipLaunchKernelGGL(prefill_scan_kernel, dim3(B), dim3(1024), 0, st, p);
   if (K > 0) {
     hipLaunchKernelGGL(prefill_scatter_kernel, dim3(L.ntiles_cap, B), dim3(kPfTQ), 0, st, p);

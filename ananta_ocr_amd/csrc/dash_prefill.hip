@@ -240,10 +240,14 @@ __device__ __forceinline__ void load_row_slots(const PrefillArgs& a, int64_t row
 // tile kernel), otherwise its pairs are "sparse" (kind 2) and reserve a range of
 // the block's pair list.  Duplicate and unusable slots get kind 0 (first slot of a
 // block wins).  Slots are handled in groups of 16 in registers; every slot's id
-// (0 where not kept) goes to LDS for the dedup of later groups and the kinds.
+// (0 where not kept) goes to LDS for the kinds.  More than 16 slots (WIDE): a bit per block
+// and row tells which blocks the row's earlier slots named; comparing every slot with all
+// earlier ones, by LDS reads, took 178 us of the 64-slot plan of 2 x 2,730 rows.
+template <bool WIDE>
 __global__ __launch_bounds__(kPfTQ) void prefill_plan_kernel(PrefillArgs a) {
   __shared__ int32_t sCnt[kPfMaxBlocks];
-  __shared__ int16_t sId[kPfMaxSlots][kPfTQ];      // every slot's block id, per row
+  __shared__ int16_t sId[WIDE ? kPfMaxSlots : kPfMaxK][kPfTQ];   // every slot's block id, per row
+  __shared__ uint32_t sSeen[WIDE ? kPfMaxBlocks / 32 : 1][kPfTQ];
   const int b = blockIdx.y, tid = threadIdx.x;
   const int len = seq_len(a, b);
   const int t0 = blockIdx.x * kPfTQ;
@@ -251,6 +255,8 @@ __global__ __launch_bounds__(kPfTQ) void prefill_plan_kernel(PrefillArgs a) {
   const int klen = key_len(a, b);
   const int nblk = (klen + a.bs - 1) / a.bs;
   for (int i = tid; i < nblk; i += kPfTQ) sCnt[i] = 0;
+  if (WIDE)
+    for (int i = 0; i < (nblk + 31) / 32; ++i) sSeen[i][tid] = 0u;
   __syncthreads();
   const int t = t0 + tid;
   const int64_t row = row0(a, b) + t;
@@ -266,15 +272,22 @@ __global__ __launch_bounds__(kPfTQ) void prefill_plan_kernel(PrefillArgs a) {
       for (int s = 0; s < kPfMaxK; ++s) {
         bool ok = ((vmask >> s) & 1u) && c[s] >= 0 && c[s] < nblk && c[s] * a.bs < ls &&
                   (c[s] + 1) * a.bs > km;
+        if (WIDE) {
+          if (ok) {
+            uint32_t& w = sSeen[c[s] >> 5][tid];
+            const uint32_t seen = w, bit = 1u << (c[s] & 31);
+            ok = !(seen & bit);
+            w = seen | bit;
+          }
+        } else {
 #pragma unroll
-        for (int u = 0; u < s; ++u) ok = ok && !(((keep_mask >> u) & 1u) && c[u] == c[s]);
-        for (int u = 0; ok && u < g0; ++u)
-          ok = !(((keep_all >> u) & 1ull) && sId[u][tid] == c[s]);
+          for (int u = 0; u < s; ++u) ok = ok && !(((keep_mask >> u) & 1u) && c[u] == c[s]);
+        }
         if (ok) {
           keep_mask |= 1u << s;
           atomicAdd(&sCnt[c[s]], 1);
         }
-        if (g0 + s < kPfMaxSlots) sId[g0 + s][tid] = (int16_t)(ok ? c[s] : 0);
+        if (g0 + s < (WIDE ? kPfMaxSlots : kPfMaxK)) sId[g0 + s][tid] = (int16_t)(ok ? c[s] : 0);
       }
       keep_all |= (uint64_t)keep_mask << g0;
     }
@@ -323,6 +336,13 @@ __global__ __launch_bounds__(kPfTQ) void prefill_plan_kernel(PrefillArgs a) {
       for (int s = 0; s < a.K; ++s) a.kind[row * a.K + s] = (uint8_t)kind_of(s);
     }
   }
+}
+
+inline void launch_plan(const PrefillArgs& a, int ntiles, hipStream_t st) {
+  if (a.K > kPfMaxK)
+    hipLaunchKernelGGL(prefill_plan_kernel<true>, dim3(ntiles, a.B), dim3(kPfTQ), 0, st, a);
+  else
+    hipLaunchKernelGGL(prefill_plan_kernel<false>, dim3(ntiles, a.B), dim3(kPfTQ), 0, st, a);
 }
 
 // ---------------------------------------------------------------------------
@@ -1882,7 +1902,7 @@ extern "C" int dash_attn_prefill(
     const int ncount = (int)((L.err - L.count) / 4) + 1;  // block counters, arrival, error
     hipLaunchKernelGGL(prefill_clear_kernel, dim3((ncount + 255) / 256), dim3(256), 0, st,
                        a.blk_count, ncount);
-    hipLaunchKernelGGL(prefill_plan_kernel, dim3(ntiles, B), dim3(kPfTQ), 0, st, a);
+    launch_plan(a, ntiles, st);
     hipLaunchKernelGGL(prefill_scan_kernel, dim3(B), dim3(1024), 0, st, a);
     hipLaunchKernelGGL(prefill_scatter_kernel, dim3(ntiles, B), dim3(kPfTQ), 0, st, a);
     hipLaunchKernelGGL(prefill_sparse_kernel<128>, dim3(L.chunk_cap * H * B), dim3(256), 0, st, a);
@@ -2018,7 +2038,7 @@ extern "C" int dash_attn_prefill_backward(
     const int ncount = (int)((L.P.err - L.P.count) / 4) + 1;
     hipLaunchKernelGGL(prefill_clear_kernel, dim3((ncount + 255) / 256), dim3(256), 0, st,
                        p.blk_count, ncount);
-    hipLaunchKernelGGL(prefill_plan_kernel, dim3(p.ntiles, B), dim3(kPfTQ), 0, st, p);
+    launch_plan(p, p.ntiles, st);
     hipLaunchKernelGGL(prefill_scan_kernel, dim3(B), dim3(1024), 0, st, p);
     hipLaunchKernelGGL(prefill_scatter_kernel, dim3(p.ntiles, B), dim3(kPfTQ), 0, st, p);
   }
