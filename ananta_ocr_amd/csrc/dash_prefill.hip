@@ -1753,8 +1753,14 @@ namespace dash {
 // scaled fp16 dQ partials with their scales (four 32-dim pieces a row), delta.
 struct BwdLayout {
   PlanLayout P;
-  int64_t pdb, pdq, pdqs, delta, total;
+  int64_t pdb, pdq, pdqs, delta, items, nitems, sparts, pkv, total;
+  int nstage, part_steps, item_cap, slot_cap;
 };
+// Steps of a part of a key-major stage, at least; a stage's window steps count double where
+// they are more, so that the stages in parts are those of many pairs.  A third of a CU's even
+// share of the pairs' steps, 24 to 128: the heaviest stages start first, so that such parts
+// still end together, and a part's start and its 64 KB of sums cost about two steps.
+constexpr int kBwMinSteps = 24, kBwMaxSteps = 128;
 
 inline BwdLayout bwd_layout(int B, int H, int S_max, int64_t rows, int K, int D, int nblk_cap,
                             int bs) {
@@ -1766,6 +1772,21 @@ inline BwdLayout bwd_layout(int B, int H, int S_max, int64_t rows, int K, int D,
   L.pdq = o; o = align256(o + L.P.ppos * H * nsub * (int64_t)D * 2);
   L.pdqs = o; o = align256(o + L.P.ppos * H * nsub * 4 * 4);
   L.delta = o; o = align256(o + rows * H * 4);
+  L.nstage = (int)(((int64_t)nblk_cap * bs + kBwIT - 1) / kBwIT);
+  // stages that take a block's pairs
+  const int64_t per = bs <= kBwIT ? 1 : bs % kBwIT == 0 ? nsub : nsub + 1;
+  const int64_t est = H * (per * rows * K / kBwIT + rows / kBwIT + B) / (256 * 3);
+  L.part_steps = (int)std::min<int64_t>(std::max<int64_t>(est, kBwMinSteps), kBwMaxSteps);
+  // a stage in parts of X steps has more than X / 2 steps of pairs (r), so at most
+  // (r + X / 2) / X + 1 <= 4 r / X parts
+  const int64_t pair_steps = K > 0 ? per * ((int64_t)S_max * K / kBwIT + nblk_cap) : 0;
+  const int64_t slots = 4 * pair_steps / L.part_steps + 1;
+  L.slot_cap = (int)slots;
+  L.item_cap = (int)(L.nstage + 2 * pair_steps / L.part_steps + 1);   // parts - 1 < 2 r / X
+  L.items = o; o = align256(o + (int64_t)B * L.item_cap * 16);
+  L.nitems = o; o = align256(o + (int64_t)B * 4);
+  L.sparts = o; o = align256(o + (int64_t)B * L.nstage * 8);
+  L.pkv = o; o = align256(o + (int64_t)B * H * L.slot_cap * 2 * kBwIT * D * 4);
   L.total = o;
   return L;
 }
@@ -2010,7 +2031,13 @@ extern "C" int dash_attn_prefill_backward(
   a.dbias = dbias;
   a.scale = scale;
   a.nsub = (block_size + kBwIT - 1) / kBwIT;
-  a.nstage = (int)(((int64_t)nblk_cap * block_size + kBwIT - 1) / kBwIT);
+  a.nstage = L.nstage;
+  a.part_steps = std::max(L.part_steps, 2 * ((kBwIT - 2 + local_window) / kBwIT + 1));
+  a.item_cap = L.item_cap; a.slot_cap = L.slot_cap;
+  a.items = (int4*)(w + L.items);
+  a.n_items = (int32_t*)(w + L.nitems);
+  a.stage_parts = (int2*)(w + L.sparts);
+  a.part_kv = (float*)(w + L.pkv);
   a.delta = (float*)(w + L.delta);
   a.part_db = (float*)(w + L.pdb);
   a.part_dq = (_Float16*)(w + L.pdq);
@@ -2042,7 +2069,10 @@ extern "C" int dash_attn_prefill_backward(
     hipLaunchKernelGGL(prefill_scan_kernel, dim3(B), dim3(1024), 0, st, p);
     hipLaunchKernelGGL(prefill_scatter_kernel, dim3(p.ntiles, B), dim3(kPfTQ), 0, st, p);
   }
-  hipLaunchKernelGGL(bwd_kv_kernel, dim3(stream_stage_grid(B * H, a.nstage)), dim3(512), 0, st, a);
+  hipLaunchKernelGGL(bwd_items_kernel, dim3(B), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(bwd_kv_kernel, dim3(stream_stage_grid(B * H, a.item_cap)), dim3(512), 0, st, a);
+  if (K > 0)
+    hipLaunchKernelGGL(bwd_sum_kernel, dim3(4 * a.nstage, H, B), dim3(256), 0, st, a);
   hipLaunchKernelGGL(bwd_q_kernel, dim3(p.ntiles * H * B), dim3(256), 0, st, a);
   if (dbias && K > 0 && total_rows > 0)
     hipLaunchKernelGGL(bwd_dbias_kernel, dim3((unsigned)((total_rows * K + 255) / 256)), dim3(256), 0,

@@ -57,6 +57,14 @@ struct BwdArgs {
   float* part_db;                         // [H, ppos, nsub] fp32
   float scale;                            // natural softmax scale
   int nstage;                             // 64-key stages per sequence (of nblk_cap blocks)
+  // key-major work list (bwd_items_kernel): a stage of more than part_steps steps is cut
+  // into parts, whose dK and dV go to part_kv in fp32 and are added by bwd_sum_kernel
+  int part_steps;
+  int item_cap, slot_cap;                 // items and part slots per sequence
+  int4* items;                            // [B, item_cap] stage, part, parts, first slot
+  int32_t* n_items;                       // [B]
+  int2* stage_parts;                      // [B, nstage] first slot, parts (0: nothing to add)
+  float* part_kv;                         // [B, H, slot_cap, 2, 64, 128] dK (not scaled), dV
   int nsub;                               // 64-key stages per block (1 for blocks <= 64 keys)
 };
 
@@ -261,6 +269,73 @@ __device__ __forceinline__ void stage_rows8r(bf16* sX, int wv, int lane, const b
                                      16, 0, 0);
 }
 
+// The steps of a key-major stage: n_win 64-query steps of the window band, then the routed
+// pairs of the stage's (at most two) blocks, 64 at a time.
+struct KvSteps {
+  int n_win, rs0, n, np0, np1, ch00, ch01;
+};
+__device__ __forceinline__ KvSteps kv_steps(const PrefillArgs& p, int b, int len, int j0) {
+  KvSteps k = {};
+  const int t_end = min(j0 + kBwIT - 1 + p.lw - 1, len - 1);
+  k.n_win = t_end >= j0 ? (t_end - j0) / kBwIT + 1 : 0;
+  const int c_first = j0 / p.bs;
+  const int c_last = p.blk_count ? min(j0 + kBwIT - 1, len - 1) / p.bs : c_first - 1;  // <= c_first + 1
+  if (c_last >= c_first) {
+    k.np0 = p.blk_count[(int64_t)b * p.nblk_cap + c_first];
+    k.ch00 = p.blk_chunk[(int64_t)b * p.nblk_cap + c_first];
+  }
+  if (c_last > c_first) {
+    k.np1 = p.blk_count[(int64_t)b * p.nblk_cap + c_first + 1];
+    k.ch01 = p.blk_chunk[(int64_t)b * p.nblk_cap + c_first + 1];
+  }
+  k.rs0 = (k.np0 + kBwIT - 1) / kBwIT;
+  k.n = k.n_win + k.rs0 + (k.np1 + kBwIT - 1) / kBwIT;
+  return k;
+}
+
+// Work list of the key-major kernel, one work-group per sequence: its stages in order, each
+// in ceil(steps / part_steps) parts.  A block that most queries route to (the first blocks,
+// where zero priors tie) has hundreds of steps, which one work-group took alone while the
+// other CUs ran dry.
+__global__ __launch_bounds__(256) void bwd_items_kernel(BwdArgs a) {
+  __shared__ int sSum[2][4];
+  const PrefillArgs& p = a.p;
+  const int b = blockIdx.x, tid = threadIdx.x, lane = wave_lane(), wv = tid / kWave;
+  const int len = seq_len(p, b);
+  int item0 = 0, slot0 = 0;
+  for (int s0 = 0; s0 < a.nstage; s0 += 256) {
+    const int stage = s0 + tid, j0 = stage * kBwIT;
+    int parts = 0;
+    if (stage < a.nstage && j0 / p.bs * p.bs < len)
+      parts = max(1, (kv_steps(p, b, len, j0).n + a.part_steps - 1) / a.part_steps);
+    const int slots = parts > 1 ? parts : 0;
+    int xi = parts, xs = slots;            // inclusive prefixes over the wavefront
+#pragma unroll
+    for (int m = 1; m < kWave; m <<= 1) {
+      const int yi = __shfl_up(xi, m, kWave), ys = __shfl_up(xs, m, kWave);
+      if (lane >= m) { xi += yi; xs += ys; }
+    }
+    if (lane == kWave - 1) { sSum[0][wv] = xi; sSum[1][wv] = xs; }
+    __syncthreads();
+    int ti = 0, ts = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      if (w < wv) { xi += sSum[0][w]; xs += sSum[1][w]; }
+      ti += sSum[0][w];
+      ts += sSum[1][w];
+    }
+    __syncthreads();
+    const int fi = item0 + xi - parts, fs = slot0 + xs - slots;
+    for (int q = 0; q < parts; ++q)
+      if (fi + q < a.item_cap)             // always, as are the slots below slot_cap
+        a.items[(int64_t)b * a.item_cap + fi + q] = make_int4(stage, q, parts, fs);
+    if (stage < a.nstage) a.stage_parts[(int64_t)b * a.nstage + stage] = make_int2(fs, slots);
+    item0 += ti;
+    slot0 += ts;
+  }
+  if (tid == 0) a.n_items[b] = min(item0, a.item_cap);
+}
+
 // Key-major kernel, eight wavefronts: wavefront (kh, qc, dh) = (wv % 2, wv / 2 % 2,
 // wv / 4) owns keys 32 kh .. + 31 of the stage, queries 32 qc .. + 31 of a step and
 // head dims 64 dh .. + 63 of dK and dV, so that two wavefronts fit on a SIMD.  Per
@@ -301,12 +376,14 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_kernel(BwdArgs a) {
   // stage) and contiguous per XCD instead, the heavy stages of some heads started
   // last: 2.61 -> 2.04 ms), while neighbouring stages, whose window bands overlap,
   // share one L2.
-  int bh, stage;
-  if (!stream_stage_item((int)blockIdx.x, p.B * p.H, a.nstage, bh, stage)) return;
+  int bh, item;
+  if (!stream_stage_item((int)blockIdx.x, p.B * p.H, a.item_cap, bh, item)) return;
   const int h = bh % p.H, b = bh / p.H;
+  if (item >= a.n_items[b]) return;
+  const int4 it = a.items[(int64_t)b * a.item_cap + item];
+  const int nparts = it.z;
   const int len = seq_len(p, b);
-  const int j0 = stage * kBwIT;
-  if (j0 / p.bs * p.bs >= len) return;
+  const int j0 = it.x * kBwIT;
   const int sub = (j0 % p.bs) / kBwIT;
   const int tid = threadIdx.x, lane = wave_lane(), wv = tid / kWave;
   const int kh = wv & 1, qc = (wv >> 1) & 1, dh = wv >> 2, hl = lane >> 5, n = lane & 31;
@@ -322,21 +399,13 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_kernel(BwdArgs a) {
   stage_rows8(sV, wv, lane, [&](int r) { return vb + (int64_t)min(j0 + r, len - 1) * p.v_st; });
 
   const int LW = p.lw, bs = p.bs;
-  const int t_end = min(j0 + kBwIT - 1 + LW - 1, len - 1);
-  const int n_win = t_end >= j0 ? (t_end - j0) / kBwIT + 1 : 0;
   const int c_first = j0 / bs;
-  const int c_last = p.blk_count ? min(j0 + kBwIT - 1, len - 1) / bs : c_first - 1;  // <= c_first + 1
-  int np0 = 0, np1 = 0, ch00 = 0, ch01 = 0;
-  if (c_last >= c_first) {
-    np0 = p.blk_count[(int64_t)b * p.nblk_cap + c_first];
-    ch00 = p.blk_chunk[(int64_t)b * p.nblk_cap + c_first];
-  }
-  if (c_last > c_first) {
-    np1 = p.blk_count[(int64_t)b * p.nblk_cap + c_first + 1];
-    ch01 = p.blk_chunk[(int64_t)b * p.nblk_cap + c_first + 1];
-  }
-  const int rs0 = (np0 + kBwIT - 1) / kBwIT;
-  const int n_steps = n_win + rs0 + (np1 + kBwIT - 1) / kBwIT;
+  const KvSteps ks_ = kv_steps(p, b, len, j0);
+  const int n_win = ks_.n_win, rs0 = ks_.rs0;
+  const int np0 = ks_.np0, np1 = ks_.np1, ch00 = ks_.ch00, ch01 = ks_.ch01;
+  // this part's steps [s_first, n_steps)
+  const int s_first = (int)((int64_t)ks_.n * it.y / nparts);
+  const int n_steps = (int)((int64_t)ks_.n * (it.y + 1) / nparts);
 
   auto pair_of = [&](int u) -> int {
     const int v = u - n_win;
@@ -400,13 +469,13 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_kernel(BwdArgs a) {
   float* const xs = sX[wv];                // own staging area
 
   int pid_next = -1;
-  if (n_steps > 0) {
+  if (n_steps > s_first) {
     if (wv == 0) {
-      const int pid0 = n_win > 0 ? -1 : pair_of(0);
-      pid_next = n_steps > 1 && n_win <= 1 ? pair_of(1) : -1;
-      meta_store(0, meta_load(0, pid0), sM[0]);
-      sRow[0][tid & 31][tid >> 5] = row_of(0, pid0);
-      if (n_steps > 1) sRow[1][tid & 31][tid >> 5] = row_of(1, pid_next);
+      const int pid0 = s_first < n_win ? -1 : pair_of(s_first);
+      pid_next = s_first + 1 < n_steps && s_first + 1 >= n_win ? pair_of(s_first + 1) : -1;
+      meta_store(s_first, meta_load(s_first, pid0), sM[0]);
+      sRow[0][tid & 31][tid >> 5] = row_of(s_first, pid0);
+      if (s_first + 1 < n_steps) sRow[1][tid & 31][tid >> 5] = row_of(s_first + 1, pid_next);
     }
     __syncthreads();
     const int2 rw = *(const int2*)&sRow[0][4 * wv + (lane >> 4)][0];
@@ -640,13 +709,13 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_kernel(BwdArgs a) {
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
   };
-  int s = 0;
+  int s = s_first;
   for (; s + 1 < n_steps; s += 2) {
     step(s, std::integral_constant<int, 0>{});
     step(s + 1, std::integral_constant<int, 1>{});
   }
   if (s < n_steps) step(s, std::integral_constant<int, 0>{});
-  store_pending((n_steps - 1) & 1);
+  store_pending((n_steps - s_first - 1) & 1);
 
   // ---- dK and dV: the two query chunks' sums (16 KB per (kh, dh) pair) ----
   const int ri = kh + 2 * dh;
@@ -661,6 +730,27 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_kernel(BwdArgs a) {
       }
   }
   __syncthreads();
+  if (nparts > 1) {                        // this part's share, added by bwd_sum_kernel
+    if (qc == 0) {
+      float* const pk = a.part_kv + ((((int64_t)b * p.H + h) * a.slot_cap + it.w + it.y) * 2 * kBwIT +
+                                     32 * kh + n) * D + 64 * dh + 4 * hl;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          float wk[4], wvv[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int r = 4 * g + j;
+            wk[j] = acc_dk[t][r] + red[(t * 16 + r) * kWave + lane];
+            wvv[j] = acc_dv[t][r] + red[((2 + t) * 16 + r) * kWave + lane];
+          }
+          *(float4*)(pk + 32 * t + 8 * g) = make_float4(wk[0], wk[1], wk[2], wk[3]);
+          *(float4*)(pk + kBwIT * D + 32 * t + 8 * g) = make_float4(wvv[0], wvv[1], wvv[2], wvv[3]);
+        }
+    }
+    return;
+  }
   if (qc == 0 && key < len) {
     bf16* dkp = seq_base(a.dk, p.cu, b, a.dk_sb, a.dk_st) + (int64_t)h * a.dk_sh + (int64_t)key * a.dk_st;
     bf16* dvp = seq_base(a.dv, p.cu, b, a.dv_sb, a.dv_st) + (int64_t)h * a.dv_sh + (int64_t)key * a.dv_st;
@@ -678,6 +768,39 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_kernel(BwdArgs a) {
         *(bf16x4*)(dkp + 64 * dh + 32 * t + 8 * g + 4 * hl) = wk;
         *(bf16x4*)(dvp + 64 * dh + 32 * t + 8 * g + 4 * hl) = wvv;
       }
+  }
+}
+
+// dK and dV of the stages in parts: the parts' shares in order, in fp32.  A work-group takes
+// a quarter of one stage's dK and dV.
+__global__ __launch_bounds__(256) void bwd_sum_kernel(BwdArgs a) {
+  constexpr int D = 128;
+  const PrefillArgs& p = a.p;
+  const int stage = blockIdx.x >> 2, h = blockIdx.y, b = blockIdx.z;
+  const int2 sp = a.stage_parts[(int64_t)b * a.nstage + stage];
+  if (sp.y == 0) return;
+  const int len = seq_len(p, b);
+  const float4* src = (const float4*)(a.part_kv + (((int64_t)b * p.H + h) * a.slot_cap + sp.x) * 2 * kBwIT * D);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int e = (blockIdx.x & 3) * 1024 + u * 256 + threadIdx.x;   // float4 of the 2 x 64 x 32
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int q = 0; q < sp.y; ++q) {
+      const float4 x = src[(int64_t)q * 2 * kBwIT * (D / 4) + e];
+      s.x += x.x; s.y += x.y; s.z += x.z; s.w += x.w;
+    }
+    const int key = stage * kBwIT + (e >> 5) % kBwIT, d = (e & 31) * 4;
+    if (key >= len) continue;
+    const bool isv = e >= kBwIT * (D / 4);
+    const float c = isv ? 1.f : a.scale;
+    bf16* o = isv ? seq_base(a.dv, p.cu, b, a.dv_sb, a.dv_st) + (int64_t)h * a.dv_sh + (int64_t)key * a.dv_st
+                  : seq_base(a.dk, p.cu, b, a.dk_sb, a.dk_st) + (int64_t)h * a.dk_sh + (int64_t)key * a.dk_st;
+    bf16x4 w;
+    w[0] = (bf16)(s.x * c);
+    w[1] = (bf16)(s.y * c);
+    w[2] = (bf16)(s.z * c);
+    w[3] = (bf16)(s.w * c);
+    *(bf16x4*)(o + d) = w;
   }
 }
 
