@@ -76,10 +76,17 @@ __global__ __launch_bounds__(256) void kbar_kernel(
 constexpr int kKbD = 128;
 constexpr int kKbMaxBs = 64;
 
+// Summaries written to a page pool (rows > 0): the block's page names the row; blocks from
+// first[b] / div on.
+struct KbarPages {
+  const int32_t* first;
+  int div, rows;
+};
+
 __global__ __launch_bounds__(256) void kbar128_kernel(
     const float* __restrict__ idx_k, SeqLayout lay, const int32_t* __restrict__ cu,
     const int32_t* __restrict__ lens, const float* __restrict__ head_cls, int S, int bs,
-    int tail_only, float inv_sqrt_d, float* __restrict__ kbar, int64_t kb_sb) {
+    int tail_only, float inv_sqrt_d, float* __restrict__ kbar, int64_t kb_sb, KbarPages pg) {
   __shared__ float4 s_k[kKbMaxBs][kKbD / 4 + 1];
   __shared__ float s_w[kKbMaxBs];
   __shared__ float4 s_part[8][kKbD / 4];
@@ -89,6 +96,13 @@ __global__ __launch_bounds__(256) void kbar128_kernel(
   const int c = tail_only ? (len - 1) / bs : (int)blockIdx.x;
   const int t0 = c * bs;
   if (t0 >= len) return;
+  float* dst = kbar + (int64_t)b * kb_sb + (int64_t)c * kKbD;
+  if (pg.rows > 0) {
+    if (c < pg.first[b] / pg.div) return;
+    const int page = lay.table[(int64_t)b * lay.table_stride + c];
+    if (page < 0 || page >= pg.rows) return;
+    dst = kbar + (int64_t)page * kKbD;
+  }
   const int n = min(bs, len - t0);
   const int tid = threadIdx.x, lane = wave_lane();
 
@@ -149,7 +163,7 @@ __global__ __launch_bounds__(256) void kbar128_kernel(
 #pragma unroll
     for (int g = 0; g < 8; ++g) acc += sp[g * kKbD + tid];
     if (!(fabsf(acc) <= 3.402823466e38f)) acc = 0.f;   // nan_to_num(nan/inf -> 0)
-    kbar[(int64_t)b * kb_sb + (int64_t)c * kKbD + tid] = acc;
+    dst[tid] = acc;
   }
 }
 
@@ -296,7 +310,8 @@ __global__ __launch_bounds__(256) void scores_mfma_kernel(
     const float* __restrict__ idx_q, SeqLayout lay_q, const int32_t* __restrict__ cu_q, int Lq,
     const int32_t* __restrict__ q_pos, const float* __restrict__ kbar, int64_t kb_sb,
     const int32_t* __restrict__ cu_k, const int32_t* __restrict__ lens_k, int S, int bs,
-    int local_blocks, int nblk_cap, float inv_sqrt_d, float* __restrict__ z, int64_t z_stride) {
+    int local_blocks, int nblk_cap, float inv_sqrt_d, float* __restrict__ z, int64_t z_stride,
+    const int32_t* __restrict__ kb_table, int64_t kb_ts, int kb_rows) {
   __shared__ __attribute__((aligned(16))) bf16 sK[3][kSmBlk * 128];
   __shared__ int sLim[kSmRows];
   const int b = blockIdx.z;
@@ -343,7 +358,13 @@ __global__ __launch_bounds__(256) void scores_mfma_kernel(
     const int e = (tid + 256 * j) * 4;          // element of the 64 x 128 tile
     const int n = e / 128, k = e % 128;
     kv[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (c0 + n < nblk_cap) kv[j] = *(const float4*)(kbar + (int64_t)b * kb_sb + (int64_t)(c0 + n) * 128 + k);
+    if (c0 + n < nblk_cap) {
+      // a page pool (kb_table): the block's row is its page; entries past a sequence's
+      // blocks may hold anything and their scores are masked
+      const int64_t row = kb_table ? min(max(kb_table[(int64_t)b * kb_ts + c0 + n], 0), kb_rows - 1)
+                                   : c0 + n;
+      kv[j] = *(const float4*)(kbar + (int64_t)b * kb_sb + row * 128 + k);
+    }
   }
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
@@ -1252,7 +1273,7 @@ extern "C" int dash_kbar(const float* idx_k, int64_t ik_sb, int64_t ik_st, int64
   if (d == kKbD && block_size <= kKbMaxBs && aligned) {
     hipLaunchKernelGGL(kbar128_kernel, grid, dim3(256), 0, (hipStream_t)stream, idx_k, lay,
                        cu_seqlens, seq_lens, head_cls, S, block_size, tail_only,
-                       (float)(1.0 / sqrt((double)d)), kbar, kb_sb);
+                       (float)(1.0 / sqrt((double)d)), kbar, kb_sb, KbarPages{});
     return launch_status();
   }
   hipLaunchKernelGGL(kbar_kernel, grid, dim3(256), 0, (hipStream_t)stream, idx_k, lay,
@@ -1279,13 +1300,73 @@ extern "C" int dash_block_scores(const float* idx_q, int64_t iq_sb, int64_t iq_s
     dim3 g2((Lq + kSmRows - 1) / kSmRows, (nblk_cap + kSmBlk - 1) / kSmBlk, B);
     hipLaunchKernelGGL(scores_mfma_kernel, g2, dim3(256), 0, (hipStream_t)stream, idx_q, lay, cu_q,
                        Lq, q_pos, kbar, kb_sb, cu_k, lens_k, S, block_size, local_blocks, nblk_cap,
-                       (float)(1.0 / sqrt((double)d)), z, z_stride);
+                       (float)(1.0 / sqrt((double)d)), z, z_stride, (const int32_t*)nullptr,
+                       (int64_t)0, 0);
     return launch_status();
   }
   auto kern = vec ? scores_kernel<true> : scores_kernel<false>;
   hipLaunchKernelGGL(kern, grid, dim3(256), 0, (hipStream_t)stream, idx_q, lay, cu_q,
                      Lq, q_pos, kbar, kb_sb, cu_k, lens_k, S, d, block_size, local_blocks,
                      nblk_cap, (float)(1.0 / sqrt((double)d)), z, z_stride);
+  return launch_status();
+}
+
+// ---------------------------------------------------------------------------
+// Router inputs of an extend step
+// ---------------------------------------------------------------------------
+namespace dash {
+// Position and block count of every query row: row cu[b] + i is position ctx[b] + i of
+// sequence b.
+__global__ __launch_bounds__(256) void extend_rows_kernel(const int32_t* __restrict__ cu,
+                                                          const int32_t* __restrict__ ctx,
+                                                          const int32_t* __restrict__ lens, int B,
+                                                          int T, int bs, int32_t* __restrict__ q_pos,
+                                                          int32_t* __restrict__ row_nblk) {
+  const int r = blockIdx.x * 256 + threadIdx.x;
+  if (r >= T) return;
+  int b = 0, hi = B;                       // the last sequence b with cu[b] <= r
+  while (hi - b > 1) {
+    const int mid = (b + hi) >> 1;
+    if (cu[mid] <= r) b = mid; else hi = mid;
+  }
+  q_pos[r] = ctx[b] + r - cu[b];
+  row_nblk[r] = (lens[b] + bs - 1) / bs;
+}
+}  // namespace dash
+
+extern "C" int dash_extend_scores(const float* idx_q, int64_t iq_st, const float* idx_k,
+                                  int64_t ik_st, int64_t ik_sp, const float* head_cls,
+                                  const int32_t* cu_seqlens_q, const int32_t* context_lens,
+                                  const int32_t* seq_lens, const int32_t* block_table,
+                                  int64_t table_stride, float* pool, int pool_rows, int B, int T,
+                                  int max_query_len, int nblk, int d, int block_size,
+                                  int local_blocks, int32_t* q_pos, int32_t* row_nblk, float* z,
+                                  int64_t z_stride, void* stream) {
+  using namespace dash;
+  if (!idx_q || !idx_k || !head_cls || !cu_seqlens_q || !context_lens || !seq_lens || !block_table ||
+      !pool || !q_pos || !row_nblk || !z || B < 0 || T < 0 || max_query_len < 0 || nblk < 0 ||
+      pool_rows <= 0)
+    return kErrInvalid;
+  if (d != kKbD || block_size <= 0 || block_size > kKbMaxBs || iq_st % 4 != 0 || ik_st % 4 != 0 ||
+      ik_sp % 4 != 0 || (uintptr_t)idx_q % 16 != 0 || (uintptr_t)idx_k % 16 != 0 ||
+      (uintptr_t)head_cls % 16 != 0 || (uintptr_t)pool % 16 != 0 || B > 65535)
+    return kErrUnsupported;
+  if (B == 0 || nblk == 0) return kOk;
+  hipStream_t st = (hipStream_t)stream;
+  const float inv = (float)(1.0 / sqrt((double)d));
+  const SeqLayout lk{nullptr, block_table, table_stride, 0, ik_sp, ik_st, block_size};
+  hipLaunchKernelGGL(kbar128_kernel, dim3(nblk, B), dim3(256), 0, st, idx_k, lk,
+                     (const int32_t*)nullptr, seq_lens, head_cls, nblk * block_size, block_size, 0, inv,
+                     pool, (int64_t)0, KbarPages{context_lens, block_size, pool_rows});
+  if (T == 0 || max_query_len == 0) return launch_status();
+  hipLaunchKernelGGL(extend_rows_kernel, dim3((T + 255) / 256), dim3(256), 0, st, cu_seqlens_q,
+                     context_lens, seq_lens, B, T, block_size, q_pos, row_nblk);
+  const SeqLayout lq{cu_seqlens_q, nullptr, 0, 0, 0, iq_st, 1};
+  dim3 grid((max_query_len + kSmRows - 1) / kSmRows, (nblk + kSmBlk - 1) / kSmBlk, B);
+  hipLaunchKernelGGL(scores_mfma_kernel, grid, dim3(256), 0, st, idx_q, lq, cu_seqlens_q,
+                     max_query_len, q_pos, pool, (int64_t)0, (const int32_t*)nullptr, seq_lens,
+                     nblk * block_size, block_size, local_blocks, nblk, inv, z, z_stride, block_table,
+                     table_stride, pool_rows);
   return launch_status();
 }
 

@@ -806,16 +806,47 @@ def attn_rows(q, k, v, idx, bias, valid, q_pos, row_seq, block_size, local_windo
     return out
 
 
-# Fewest query rows of an extend step for the block-grouped matrix-core path.  Up to 128 rows
-# both paths take the step's launch time (window 512, 16 blocks of 64, caches of 13,650 tokens:
-# 345 us row by row, 347 grouped); 256 rows 484 against 347, 2,048 rows 2,849 against 368.
-EXTEND_ROWS = 128
+def extend_scores_ok(idx_q, idx_k, pool, block_size):
+    """Whether extend_scores takes these index queries, paged index keys and k_bar pool."""
+    return (idx_q.dim() == 2 and idx_k.dim() == 3 and idx_q.shape[-1] == idx_k.shape[-1] == 128
+            and pool.shape[-1] == 128 and 0 < block_size <= 64 and pool.shape[0] > 0
+            and pool.dtype == torch.float32 and pool.is_contiguous()
+            and all(x.is_cuda and x.dtype == torch.float32 and x.stride(-1) == 1
+                    and x.data_ptr() % 16 == 0 and all(s % 4 == 0 for s in x.stride()[:-1])
+                    for x in (idx_q, idx_k)))
+
+
+def extend_scores(idx_q, idx_k, head_cls, cu_seqlens_q, context_lens, seq_lens, block_table, pool,
+                  block_size, local_blocks, max_query_len):
+    """Router inputs of an extend step (dash_extend_scores): refreshes the k_bar pool from each
+    request's boundary page on and returns the block scores z [T,P] of the query rows, their
+    positions and block counts [T] int32.  Lengths and table int32 on the GPU."""
+    _need_gpu(idx_q, idx_k, head_cls, cu_seqlens_q, context_lens, seq_lens, block_table, pool)
+    lib = _lib.load()
+    T, d = idx_q.shape
+    B, P = block_table.shape
+    zs = max(32, (P + 31) // 32 * 32)
+    dev = idx_q.device
+    z = torch.empty(T, zs, dtype=torch.float32, device=dev)
+    rows = torch.empty(2, T, dtype=torch.int32, device=dev)
+    hc = head_cls.float().contiguous()
+    if hc.data_ptr() % 16:
+        hc = hc.clone()
+    st_ = lib.dash_extend_scores(
+        _ptr(idx_q), idx_q.stride(0), _ptr(idx_k), idx_k.stride(1), idx_k.stride(0), _ptr(hc),
+        _ptr(cu_seqlens_q), _ptr(context_lens), _ptr(seq_lens), _ptr(block_table),
+        block_table.stride(0), _ptr(pool), pool.shape[0], B, T, int(max_query_len), P, d,
+        int(block_size), int(local_blocks), _ptr(rows[0]), _ptr(rows[1]), _ptr(z), zs, _stream())
+    _lib.check(st_, "dash_extend_scores")
+    return z[:, :P], rows[0], rows[1]
 
 
 def attn_extend_ok(q, k, v, K, block_size, page_size, num_blocks, scale):
-    """Whether attn_extend takes these rows (else attn_rows)."""
-    return (q.shape[0] >= EXTEND_ROWS and q.shape[2] == 128 and block_size in (32, 64)
-            and page_size == block_size and K <= 64 and num_blocks <= 2048 and scale > 0
+    """Whether attn_extend takes these rows (else attn_rows).  Any number of rows: an extend
+    step of 2 rows takes 107 us grouped and 138 row by row (caches of 13,650 tokens), of 128
+    rows 155 and 233, of 512 rows 168 and 744."""
+    return (q.shape[2] == 128 and block_size in (32, 64) and page_size == block_size
+            and 0 < K <= 64 and num_blocks <= 2048 and scale > 0
             and q.shape[0] * q.shape[1] * max(K, 1) < 2 ** 31)
 
 

@@ -109,6 +109,12 @@ class KBarPageCache:
         self._buf.index_copy_(0, tgt.reshape(-1), kb.reshape(-1, kb.shape[-1]))
 
 
+def _row_seq(cu, B, T):
+    """Sequence of each of the T packed query rows, without a host synchronisation."""
+    return torch.repeat_interleave(torch.arange(B, device=cu.device), (cu[1:] - cu[:-1]).long(),
+                                   output_size=T)
+
+
 def extend_prefill(state, q, k_cache, v_cache, idx_q, idx_k, head_cls, block_size,
                    local_blocks, idx_scale, floor, sigma, K, topm, block_table, seq_lens,
                    context_lens, cu_seqlens_q, max_query_len=None, scale=None,
@@ -140,33 +146,37 @@ def extend_prefill(state, q, k_cache, v_cache, idx_q, idx_k, head_cls, block_siz
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     dev = q.device
-    seq = seq_lens.to(device=dev, dtype=torch.int64)
-    ctx = context_lens.to(device=dev, dtype=torch.int64)
-    cu = cu_seqlens_q.to(device=dev, dtype=torch.int64)
-    state.refresh_from(idx_k, head_cls, block_size, block_table, seq, ctx // block_size)
+    seq, ctx, cu = (x.to(device=dev, dtype=torch.int32).contiguous()
+                    for x in (seq_lens, context_lens, cu_seqlens_q))
+    table = block_table.to(device=dev, dtype=torch.int32)
+    P = table.shape[1]
     max_query_len = ops._max_len(cu, max_query_len)
-    P = block_table.shape[1]
-    pages = block_table.to(torch.int64).clamp(0, state.kbar.shape[0] - 1)
-    kb_seq = state.kbar.index_select(0, pages.reshape(-1)).view(B, P, -1)
-    q_lens = cu[1:] - cu[:-1]
-    row_seq = torch.repeat_interleave(torch.arange(B, device=dev), q_lens, output_size=T)
-    rows = torch.arange(T, device=dev)
-    q_pos = (ctx.index_select(0, row_seq) + rows - cu.index_select(0, row_seq)).to(torch.int32)
-    z = ops.block_scores(idx_q.reshape(1, T, -1), kb_seq, block_size, local_blocks,
-                         q_pos=q_pos, cu_seqlens=cu, max_seqlen=max_query_len, key_lens=seq,
-                         S=P * block_size)
-    nblk_b = (seq + block_size - 1) // block_size
+    idx_q = idx_q.reshape(T, -1)
+    if ops.extend_scores_ok(idx_q, idx_k, state.kbar, block_size) and table.stride(1) == 1:
+        z, q_pos, row_nblk = ops.extend_scores(idx_q, idx_k, head_cls, cu, ctx, seq, table,
+                                               state.kbar, block_size, local_blocks, max_query_len)
+    else:
+        state.refresh_from(idx_k, head_cls, block_size, table, seq, ctx // block_size)
+        pages = table.to(torch.int64).clamp(0, state.kbar.shape[0] - 1)
+        kb_seq = state.kbar.index_select(0, pages.reshape(-1)).view(B, P, -1)
+        row_seq = _row_seq(cu, B, T)
+        q_pos = (ctx - cu[:-1]).index_select(0, row_seq) + torch.arange(T, dtype=torch.int32,
+                                                                        device=dev)
+        z = ops.block_scores(idx_q.reshape(1, T, -1), kb_seq, block_size, local_blocks,
+                             q_pos=q_pos, cu_seqlens=cu, max_seqlen=max_query_len, key_lens=seq,
+                             S=P * block_size)
+        row_nblk = ((seq + block_size - 1) // block_size).index_select(0, row_seq)
     width = max(1, min(int(K), int(topm))) if int(topm) > 0 else max(1, int(K))
     idx, bias, valid = ops.route(z, block_cand, idx_scale, floor, sigma, K, topm,
-                                 row_nblk=nblk_b.index_select(0, row_seq), width=width)
+                                 row_nblk=row_nblk, width=width)
     if ops.attn_extend_ok(q, k_cache, v_cache, idx.shape[-1], block_size, block_size, P, scale):
         out = ops.attn_extend(q, k_cache, v_cache, idx, bias, valid, seq, ctx, cu, max_query_len,
-                              block_table, block_size, local_blocks * block_size, scale,
+                              table, block_size, local_blocks * block_size, scale,
                               out_dtype=out_dtype)
     else:
-        out = ops.attn_rows(q, k_cache, v_cache, idx, bias, valid, q_pos, row_seq, block_size,
-                            local_blocks * block_size, scale, seq_lens=seq,
-                            block_table=block_table, page_size=block_size, out_dtype=out_dtype)
+        out = ops.attn_rows(q, k_cache, v_cache, idx, bias, valid, q_pos, _row_seq(cu, B, T),
+                            block_size, local_blocks * block_size, scale, seq_lens=seq,
+                            block_table=table, page_size=block_size, out_dtype=out_dtype)
     if return_routing:
         return out, (idx, bias, valid.bool()), q_pos
     return out

@@ -367,6 +367,22 @@ int dash_attn_decode(const void* q, int64_t q_sb, int64_t q_sh,
                      float scale, int nsplit, void* workspace, int64_t workspace_bytes,
                      void* stream);
 
+/*
+ * Router inputs of an extend step (kbar_all_plan, route_triton.py:576-601): the summaries
+ * of every request's blocks from context_lens[b] / block_size on, written to their pages'
+ * rows of the k_bar pool [pool_rows, 128]; the position q_pos [T] and block count
+ * row_nblk [T] of every query row; and the rows' block scores z [T, nblk] (row stride
+ * z_stride) against their request's summaries.  idx_q fp32 [T, 128]; idx_k fp32 pages
+ * [pages, block_size, 128] addressed as in dash_attn_extend.  block_size <= 64.
+ */
+int dash_extend_scores(const float* idx_q, int64_t iq_st, const float* idx_k, int64_t ik_st,
+                       int64_t ik_sp, const float* head_cls, const int32_t* cu_seqlens_q,
+                       const int32_t* context_lens, const int32_t* seq_lens,
+                       const int32_t* block_table, int64_t table_stride, float* pool,
+                       int pool_rows, int B, int T, int max_query_len, int nblk, int d,
+                       int block_size, int local_blocks, int32_t* q_pos, int32_t* row_nblk,
+                       float* z, int64_t z_stride, void* stream);
+
 /* Workspace bytes dash_attn_extend needs. */
 int dash_attn_extend_workspace_size(int B, int H, int max_query_len, int64_t T, int K, int nblk,
                                     int64_t* bytes);

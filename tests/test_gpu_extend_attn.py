@@ -11,7 +11,8 @@ import math
 import pytest
 import torch
 
-from ananta_ocr_amd import ops
+from ananta_ocr_amd import ops, pipeline
+from test_gpu_extend import test_extend_prefill_matches_per_request_oracle as _oracle_case
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -121,3 +122,40 @@ def test_extend_attention_rows_do_not_depend_on_each_other():
                           torch.tensor([0, news[1] - cut], device=DEV), news[1] - cut,
                           table[1:].to(DEV), bs, lw, scale)
     assert torch.equal(one, both[r])
+
+
+def test_extend_prefill_blocks_beyond_the_grouped_path():
+    """128-key blocks: summaries, scores and attention by the general path."""
+    _oracle_case([900, 1300, 40], [300, 0, 13], 2, 128, 2, 4, 4)
+
+
+def test_extend_scores_equal_the_general_path():
+    """Summaries in the pool, block scores, positions and block counts against kbar and
+    block_scores over per-request summaries, with an empty chunk among the requests and index
+    rows in a wider buffer."""
+    g = torch.Generator().manual_seed(1)
+    bs, lb, ctxs, news = 32, 2, [70, 5, 0, 64], [100, 0, 33, 1]
+    lens = [a + b for a, b in zip(ctxs, news)]
+    B, T, P = len(lens), sum(news), 8
+    table = torch.randperm(B * P + 3, generator=g)[:B * P].view(B, P).to(torch.int32).to(DEV)
+    ik = torch.randn(B * P + 3, bs, 256, generator=g).to(DEV)[:, :, 128:]
+    iq = torch.randn(T, 384, generator=g).to(DEV)[:, 128:256]
+    hc = torch.randn(129, generator=g).to(DEV)[1:]
+    i32 = dict(dtype=torch.int32, device=DEV)
+    ctx, ln = torch.tensor(ctxs, **i32), torch.tensor(lens, **i32)
+    cu = torch.tensor([0] + news, **i32).cumsum(0).to(torch.int32)
+    assert ops.extend_scores_ok(iq, ik, torch.zeros(B * P + 3, 128, device=DEV), bs)
+    general = pipeline.KBarPageCache(B * P + 3, 128, DEV)
+    general.refresh_from(ik, hc.clone(), bs, table, ln, ctx // bs)   # 16-byte aligned, too
+    state = pipeline.KBarPageCache(B * P + 3, 128, DEV)
+    z, q_pos, row_nblk = ops.extend_scores(iq, ik, hc, cu, ctx, ln, table, state.kbar, bs, lb,
+                                           max(news))
+    assert torch.equal(state.kbar, general.kbar)
+    seq = torch.arange(B).repeat_interleave(torch.tensor(news)).to(DEV)
+    pos = ctx[seq] + torch.arange(T, device=DEV) - cu[seq]
+    assert torch.equal(q_pos, pos.to(torch.int32))
+    assert torch.equal(row_nblk, (ln[seq] + bs - 1) // bs)
+    kb = general.kbar[table.long().reshape(-1)].view(B, P, -1)
+    ref = ops.block_scores(iq[None], kb, bs, lb, q_pos=q_pos, cu_seqlens=cu, max_seqlen=max(news),
+                           key_lens=ln, S=P * bs)
+    assert torch.equal(z, ref)
