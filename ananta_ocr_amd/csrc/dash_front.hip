@@ -36,6 +36,7 @@ struct FrontArgs {
   float* ik; int64_t ik_sb;
   float* kbar; int64_t kb_sb;
   int ntiles;
+  bf16* proj;                                 // [B * S, 256] projections (training), or null
 };
 
 struct FrontSmem {
@@ -314,6 +315,14 @@ __global__ __launch_bounds__(256, 2) void router_front_kernel(FrontArgs a) {
   for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
+      if (a.proj) {
+        const int t = t0 + fr_row(mt, i, half);
+        if (t < a.S) {
+          bf16* const o = a.proj + ((int64_t)b * a.S + t) * 256 + side * kFrD;
+          o[d0] = (bf16)acc[mt][0][i];
+          o[d1] = (bf16)acc[mt][1][i];
+        }
+      }
       const float x0 = fr_finite(fr_rb16(acc[mt][0][i]));
       const float x1 = fr_finite(fr_rb16(acc[mt][1][i]));
       acc[mt][0][i] = x0;
@@ -496,14 +505,13 @@ extern "C" int dash_router_front_pack_weights(const void* w_q, const void* w_k, 
   return front_launch_status();
 }
 
-extern "C" int dash_router_front(const void* hs, int64_t hs_sb, int64_t hs_st, int B, int S,
-                                 int hidden, const void* w_pack, const void* w_q,
-                                 const void* w_k, const float* wq_norm, const float* wk_norm,
-                                 float eps, const void* cos, const void* sin, int cs_bf16,
-                                 int64_t cs_sb, int64_t cs_st, const float* head_cls,
-                                 int block_size, float inv_sqrt_d, float* idx_q, int64_t iq_sb,
-                                 float* idx_k, int64_t ik_sb, float* kbar, int64_t kb_sb,
-                                 int nblk_cap, void* stream) {
+static int front_launch(const void* hs, int64_t hs_sb, int64_t hs_st, int B, int S, int hidden,
+                        const void* w_pack, const void* w_q, const void* w_k, const float* wq_norm,
+                        const float* wk_norm, float eps, const void* cos, const void* sin,
+                        int cs_bf16, int64_t cs_sb, int64_t cs_st, const float* head_cls,
+                        int block_size, float inv_sqrt_d, float* idx_q, int64_t iq_sb, float* idx_k,
+                        int64_t ik_sb, float* kbar, int64_t kb_sb, int nblk_cap, void* proj,
+                        void* stream) {
   using namespace dash;
   if (!hs || !w_pack || !w_q || !w_k || !wq_norm || !wk_norm || B < 0 || S < 0 || hidden <= 0)
     return kErrInvalid;
@@ -533,11 +541,37 @@ extern "C" int dash_router_front(const void* hs, int64_t hs_sb, int64_t hs_st, i
              (uintptr_t)cos % 16 == 0 && (uintptr_t)sin % 16 == 0;
   a.head_cls = head_cls; a.bs = block_size; a.inv_sqrt_d = inv_sqrt_d;
   a.iq = idx_q; a.iq_sb = iq_sb; a.ik = idx_k; a.ik_sb = ik_sb;
-  a.kbar = kbar; a.kb_sb = kb_sb;
+  a.kbar = kbar; a.kb_sb = kb_sb; a.proj = (bf16*)proj;
   a.ntiles = (S + kFrRows - 1) / kFrRows;
   const int64_t grid = (int64_t)B * a.ntiles;
   if (grid > 0x7fffffff) return kErrUnsupported;
   hipLaunchKernelGGL(router_front_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream,
                      a);
   return front_launch_status();
+}
+
+extern "C" int dash_router_front(const void* hs, int64_t hs_sb, int64_t hs_st, int B, int S,
+                                 int hidden, const void* w_pack, const void* w_q,
+                                 const void* w_k, const float* wq_norm, const float* wk_norm,
+                                 float eps, const void* cos, const void* sin, int cs_bf16,
+                                 int64_t cs_sb, int64_t cs_st, const float* head_cls,
+                                 int block_size, float inv_sqrt_d, float* idx_q, int64_t iq_sb,
+                                 float* idx_k, int64_t ik_sb, float* kbar, int64_t kb_sb,
+                                 int nblk_cap, void* stream) {
+  return front_launch(hs, hs_sb, hs_st, B, S, hidden, w_pack, w_q, w_k, wq_norm, wk_norm, eps, cos,
+                      sin, cs_bf16, cs_sb, cs_st, head_cls, block_size, inv_sqrt_d, idx_q, iq_sb,
+                      idx_k, ik_sb, kbar, kb_sb, nblk_cap, nullptr, stream);
+}
+
+extern "C" int dash_router_front_train(const void* hs, int64_t hs_sb, int64_t hs_st, int B, int S,
+                                       int hidden, const void* w_pack, const void* w_q,
+                                       const void* w_k, const float* wq_norm,
+                                       const float* wk_norm, float eps, const void* cos,
+                                       const void* sin, int cs_bf16, int64_t cs_sb, int64_t cs_st,
+                                       float* idx_q, float* idx_k, void* proj, void* stream) {
+  if (!idx_q || !idx_k || !proj) return dash::kErrInvalid;
+  const int64_t sb = (int64_t)S * dash::kFrD;
+  return front_launch(hs, hs_sb, hs_st, B, S, hidden, w_pack, w_q, w_k, wq_norm, wk_norm, eps, cos,
+                      sin, cs_bf16, cs_sb, cs_st, nullptr, 0, 0.f, idx_q, sb, idx_k, sb, nullptr, 0,
+                      0, proj, stream);
 }

@@ -2080,3 +2080,5 @@ extern "C" int dash_attn_prefill_backward(
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? kOk : (int)e;
 }
+
+#include "dash_front_bwd.h"

@@ -131,10 +131,14 @@ class GemmaRMSNorm(nn.Module):
         self.weight = nn.Parameter(torch.zeros(dim))
 
     def forward(self, x):
-        x32 = torch.nan_to_num(x.float(), nan=0.0, posinf=0.0, neginf=0.0)
-        x32 = x32 * torch.rsqrt(x32.pow(2).mean(-1, keepdim=True) + self.eps)
-        x32 = x32.clamp(-ACT_CLAMP, ACT_CLAMP)
-        return (x32 * (1.0 + self.weight.float())).clamp(-ACT_CLAMP, ACT_CLAMP).to(x.dtype)
+        return _gemma_norm(x, self.weight, self.eps)
+
+
+def _gemma_norm(x, weight, eps):
+    x32 = torch.nan_to_num(x.float(), nan=0.0, posinf=0.0, neginf=0.0)
+    x32 = x32 * torch.rsqrt(x32.pow(2).mean(-1, keepdim=True) + eps)
+    x32 = x32.clamp(-ACT_CLAMP, ACT_CLAMP)
+    return (x32 * (1.0 + weight.float())).clamp(-ACT_CLAMP, ACT_CLAMP).to(x.dtype)
 
 
 def _rotate_half(x):
@@ -147,6 +151,40 @@ def apply_rotary(q, k, cos, sin):
     cos = cos.unsqueeze(1)
     sin = sin.unsqueeze(1)
     return q * cos + _rotate_half(q) * sin, k * cos + _rotate_half(k) * sin
+
+
+def _front_train_tail(iq, ik, cos, sin):
+    """RoPE, guards and the gradient sanitizer of the normalized index queries and keys
+    [B,S,1,d] (dash_attention.py:813-821)."""
+    iq, ik = iq.transpose(1, 2), ik.transpose(1, 2)
+    if cos is not None:
+        d = iq.shape[-1]
+        iq, ik = apply_rotary(iq, ik, cos[..., :d], sin[..., :d])
+    out = []
+    for t in (iq, ik):
+        t = torch.nan_to_num(t[:, 0].float(), nan=0.0, posinf=0.0, neginf=0.0)
+        if t.requires_grad:
+            t.register_hook(_sanitize_grad)
+        out.append(t)
+    return tuple(out)
+
+
+def _front_train_ops(hs, w_q, w_k, nq, nk, cos, sin, eps):
+    """The training front end by tensor ops on the bare weights."""
+    hs = torch.nan_to_num(hs, nan=0.0, posinf=0.0, neginf=0.0)
+    iq, ik = (_gemma_norm(nn.functional.linear(hs, w), n, eps)[:, :, None]
+              for w, n in ((w_q, nq), (w_k, nk)))
+    return _front_train_tail(iq, ik, cos, sin)
+
+
+def _has_hooks(m):
+    """Whether a call of module m would run more than its class's forward: hooks (its own or
+    global ones) or a forward set on the instance."""
+    g = nn.modules.module
+    return bool("forward" in m.__dict__ or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                or m._backward_pre_hooks or g._global_forward_hooks
+                or g._global_forward_pre_hooks or g._global_backward_hooks
+                or g._global_backward_pre_hooks)
 
 
 MASK_NEG = -1.0e9
@@ -405,20 +443,22 @@ class DashAttention(nn.Module):
     def _index_qk_train(self, hidden_states, position_embeddings):
         """idx_q/idx_k [B,S,d] fp32 with autograd to the projections and norms, and
         the gradient sanitizer on both (dash_attention.py:808-821)."""
+        cos, sin = position_embeddings if position_embeddings is not None else (None, None)
+        mods = (self.q_proj, self.k_proj, self.q_norm, self.k_norm)
+        # in the library where the modules are the constructor's own, without hooks
+        if [type(m) for m in mods] == [nn.Linear, nn.Linear, GemmaRMSNorm, GemmaRMSNorm] \
+                and not any(_has_hooks(m) for m in mods) and self.q_norm.eps == self.k_norm.eps \
+                and self.q_proj.bias is None and self.k_proj.bias is None:
+            w = [m.weight for m in mods]
+            if ops.router_front_train_ok(hidden_states, *w, cos, sin):
+                return ops.router_front_train(hidden_states, *w, self.q_norm.eps, cos, sin,
+                                              _front_train_ops)
         B, S, _ = hidden_states.shape
         d = self.index_dim
         hs = torch.nan_to_num(hidden_states, nan=0.0, posinf=0.0, neginf=0.0)
-        iq = self.q_norm(self.q_proj(hs).view(B, S, 1, d)).transpose(1, 2)
-        ik = self.k_norm(self.k_proj(hs).view(B, S, 1, d)).transpose(1, 2)
-        if position_embeddings is not None:
-            cos, sin = position_embeddings
-            iq, ik = apply_rotary(iq, ik, cos[..., :d], sin[..., :d])
-        iq = torch.nan_to_num(iq[:, 0].float(), nan=0.0, posinf=0.0, neginf=0.0)
-        ik = torch.nan_to_num(ik[:, 0].float(), nan=0.0, posinf=0.0, neginf=0.0)
-        for t in (iq, ik):
-            if t.requires_grad:
-                t.register_hook(_sanitize_grad)
-        return iq, ik
+        iq = self.q_norm(self.q_proj(hs).view(B, S, 1, d))
+        ik = self.k_norm(self.k_proj(hs).view(B, S, 1, d))
+        return _front_train_tail(iq, ik, cos, sin)
 
     def _block_scores_train(self, iq, ik, position_ids, nblk):
         """Indexer scores (dash_attention.py:801-835): for query t and block c the max

@@ -369,6 +369,94 @@ def router_front(hs, w_q, w_k, nq, nk, eps, cos=None, sin=None, head_cls=None, b
     _lib.check(st_, "dash_router_front")
     return iq, (ik if idx_k_out is None else ik[:, :S]), kb
 
+def router_front_train_ok(hs, w_q, w_k, nq, nk, cos, sin):
+    """Whether router_front_train takes these inputs."""
+    if not (hs.dim() == 3 and router_front_supported(hs, w_q, w_k) and hs.shape[-1] % 128 == 0
+            and hs.numel() > 0 and nq.shape == nk.shape == (128,) and nq.is_cuda and nk.is_cuda
+            and not torch.is_autocast_enabled()):
+        return False
+    if cos is None:
+        return True
+    return (cos.dim() == 3 and cos.shape == sin.shape and cos.shape[0] in (1, hs.shape[0])
+            and cos.shape[1] == hs.shape[1] and cos.shape[2] >= 128 and cos.is_cuda and sin.is_cuda
+            and cos.dtype == sin.dtype and cos.dtype in (torch.bfloat16, torch.float32)
+            and not (cos.requires_grad or sin.requires_grad))
+
+
+class _RouterFrontFn(torch.autograd.Function):
+    """Training router front end (dash_attention.py:808-821): idx_q, idx_k [B,S,128] fp32 of
+    bf16 hidden states, with the gradient sanitizer on both."""
+
+    @staticmethod
+    def forward(ctx, hs, w_q, w_k, nq, nk, cos, sin, eps, differentiable):
+        lib = _lib.load()
+        B, S, hid = hs.shape
+        x, wq, wk = _rows(hs), w_q.contiguous(), w_k.contiguous()
+        nqf, nkf = nq.float().contiguous(), nk.float().contiguous()
+        cs, args = _front_cos_sin(cos, sin)
+        iq, ik = (torch.empty(B, S, 128, dtype=torch.float32, device=hs.device) for _ in range(2))
+        proj = torch.empty(B * S, 256, dtype=torch.bfloat16, device=hs.device)
+        pack = router_front_pack(wq, wk)
+        _lib.check(lib.dash_router_front_train(
+            _ptr(x), x.stride(0), x.stride(1), B, S, hid, _ptr(pack), _ptr(wq), _ptr(wk),
+            _ptr(nqf), _ptr(nkf), float(eps), *args, _ptr(iq), _ptr(ik), _ptr(proj), _stream()),
+            "dash_router_front_train")
+        ctx.save_for_backward(hs, w_q, w_k, nq, nk, cos, sin, proj)
+        ctx.cfg = (eps, differentiable)
+        return iq, ik
+
+    @staticmethod
+    def backward(ctx, d_iq, d_ik):
+        hs, w_q, w_k, nq, nk, cos, sin, proj = ctx.saved_tensors
+        eps, differentiable = ctx.cfg
+        need = ctx.needs_input_grad
+        if torch.is_grad_enabled():            # create_graph: by tensor ops
+            leaves = [t for t, n in zip((hs, w_q, w_k, nq, nk), need) if n]
+            got = iter(torch.autograd.grad(differentiable(hs, w_q, w_k, nq, nk, cos, sin, eps),
+                                           leaves, (d_iq, d_ik), create_graph=True))
+            return (*[next(got) if n else None for n in need[:5]], None, None, None, None)
+        lib = _lib.load()
+        B, S, hid = hs.shape
+        dev = hs.device
+        x = _rows(hs.reshape(B * S, hid))
+        wq, wk = w_q.contiguous(), w_k.contiguous()
+        nqf, nkf = nq.float().contiguous(), nk.float().contiguous()
+        cs, args = _front_cos_sin(cos, sin)
+        gq, gk = (g.float().contiguous() for g in (d_iq, d_ik))
+        dwq = torch.empty_like(wq) if need[1] else None
+        dwk = torch.empty_like(wk) if need[2] else None
+        dn = torch.empty(2, 128, dtype=torch.float32, device=dev)
+        dhs = torch.empty(B, S, hid, dtype=hs.dtype, device=dev) if need[0] else None
+        nbytes = ctypes.c_int64(0)
+        _lib.check(lib.dash_router_front_backward_workspace_size(B * S, hid, nbytes), "workspace")
+        ws = torch.empty(nbytes.value, dtype=torch.uint8, device=dev)
+        _lib.check(lib.dash_router_front_backward(
+            _ptr(proj), _ptr(gq), _ptr(gk), _ptr(nqf), _ptr(nkf), float(eps), *args, B, S, hid,
+            _ptr(x), x.stride(0), _ptr(wq), _ptr(wk), _ptr(dwq), _ptr(dwk), _ptr(dn[0]),
+            _ptr(dn[1]), _ptr(dhs), _ptr(ws), ws.numel(), _stream()), "dash_router_front_backward")
+        return (dhs, dwq, dwk, dn[0].to(nq.dtype) if need[3] else None,
+                dn[1].to(nk.dtype) if need[4] else None, None, None, None, None)
+
+
+def _front_cos_sin(cos, sin):
+    """(tensors to keep alive, C arguments) of the rotary tables [B or 1,S,>=128]."""
+    if cos is None:
+        return None, (None, None, 0, 0, 0)
+    if cos.stride(-1) != 1 or cos.stride() != sin.stride() or cos.stride(1) % 2 \
+            or cos.stride(0) % 2 or cos.data_ptr() % 8 or sin.data_ptr() % 8:
+        cos, sin = (t[..., :128].clone(memory_format=torch.contiguous_format) for t in (cos, sin))
+    return (cos, sin), (_ptr(cos), _ptr(sin), int(cos.dtype == torch.bfloat16),
+                        0 if cos.shape[0] == 1 else cos.stride(0), cos.stride(1))
+
+
+def router_front_train(hs, w_q, w_k, nq, nk, eps, cos, sin, differentiable):
+    """Index queries and keys [B,S,128] fp32 of the training front end, with autograd to the
+    hidden states, projections and norm weights; the gradients of both outputs are sanitized
+    (non-finite -> 0, clamped to +-1e4).  differentiable(hs, w_q, w_k, nq, nk, cos, sin, eps):
+    the same by tensor ops, for a graph of the gradient."""
+    return _RouterFrontFn.apply(hs, w_q, w_k, nq, nk, cos, sin, eps, differentiable)
+
+
 def route(z, cand, idx_scale, floor, sigma, K, topm, row_nblk=None, width=None):
     """Inference routing of every row of z [..., nblk] fp32.
     Returns (idx int32 [..., K'], bias fp32, valid bool) with K' = max(1, min(K, M'))."""

@@ -155,6 +155,34 @@ int dash_router_front(const void* hs, int64_t hs_sb, int64_t hs_st, int B, int S
                       const float* head_cls, int block_size, float inv_sqrt_d, float* idx_q,
                       int64_t iq_sb, float* idx_k, int64_t ik_sb, float* kbar, int64_t kb_sb,
                       int nblk_cap, void* stream);
+
+/*
+ * The same for training (dash_attention.py:808-821): idx_q and idx_k [B, S, 128] contiguous,
+ * and the bf16 projections [B * S, 256] (q then k, before the guards) that
+ * dash_router_front_backward takes.
+ */
+int dash_router_front_train(const void* hs, int64_t hs_sb, int64_t hs_st, int B, int S,
+                            int hidden, const void* w_pack, const void* w_q, const void* w_k,
+                            const float* wq_norm, const float* wk_norm, float eps,
+                            const void* cos, const void* sin, int cs_bf16, int64_t cs_sb,
+                            int64_t cs_st, float* idx_q, float* idx_k, void* proj, void* stream);
+
+/* Workspace bytes dash_router_front_backward needs for T = B * S rows. */
+int dash_router_front_backward_workspace_size(int64_t T, int hidden, int64_t* bytes);
+
+/*
+ * Gradients of dash_router_front_train from d_iq and d_ik [B, S, 128] fp32 (sanitized:
+ * non-finite -> 0, clamped to +-1e4): projection weights dw_q / dw_k bf16 [128, hidden] and
+ * hidden states dhs bf16 [B, S, hidden] (each NULL when not wanted), norm weights fp32
+ * [128].  hs rows (stride hs_st) follow each other over the batch; hidden a multiple of 128.
+ */
+int dash_router_front_backward(const void* proj, const float* d_iq, const float* d_ik,
+                               const float* wq_norm, const float* wk_norm, float eps,
+                               const void* cos, const void* sin, int cs_bf16, int64_t cs_sb,
+                               int64_t cs_st, int B, int S, int hidden, const void* hs,
+                               int64_t hs_st, const void* w_q, const void* w_k, void* dw_q,
+                               void* dw_k, float* dwq_norm, float* dwk_norm, void* dhs,
+                               void* workspace, int64_t workspace_bytes, void* stream);
 /* The q_proj / k_proj weights (bf16 [128, hidden] each, row-major) in the operand order
  * of dash_router_front: w_pack bf16 [256 * hidden]; repack when the weights change. */
 int dash_router_front_pack_weights(const void* w_q, const void* w_k, int hidden, void* w_pack,
