@@ -334,11 +334,10 @@ def _dash_decode_attend(self, router, hidden_states, q, k_all, v_all, idx_pe, po
     if dc.kbar is not None:
         # fused step: tail summary refresh + scores + routing + attention
         K = int(p["K"])
-        out, _ = ops.decode_step_fused(
+        return ops.decode_step_fused(
             q, k_all, v_all, idx_q, dc.idx_k, dc.head_cls, dc.kbar, router.block_size,
             router.local_blocks, p["idx_scale"], p["floor"], p["sigma"], K, p["topm"],
-            router._scale, cand=cand, q_pos=qpos)
-        return out
+            router._scale, cand=cand, q_pos=qpos, return_routing=False)
     # indexer stage 0: block-max scores over the raw index keys
     sc = _block_scores_infer(router, idx_q, dc.idx_k, qpos[:, None], nblk)
     topi, bias, valid = _infer_route_select(sc, None if cand is None else cand[:, None], p)

@@ -6,6 +6,7 @@ on the current HIP stream.  CPU tensors are rejected: the product has no CPU pat
 """
 
 import ctypes
+import functools
 import math
 
 import torch
@@ -20,7 +21,8 @@ def _ptr(t):
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream of the current device, as a raw handle."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _need_gpu(*ts):
@@ -30,7 +32,9 @@ def _need_gpu(*ts):
 
 
 def _i32(t):
-    return None if t is None else t.to(torch.int32).contiguous()
+    if t is None or (t.dtype == torch.int32 and t.is_contiguous()):
+        return t
+    return t.to(torch.int32).contiguous()
 
 
 def _u8(t):
@@ -51,9 +55,18 @@ def _max_len(cu, max_seqlen):
 
 def _rows(x):
     """bf16 [.., D] tensor whose feature axis is contiguous with 16-byte rows."""
-    if x.stride(-1) != 1 or any(s % 8 for s in x.stride()[:-1]) or x.data_ptr() % 16:
-        x = x.contiguous()
-    return x
+    st = x.stride()
+    ok = st[-1] == 1 and x.data_ptr() % 16 == 0
+    for s in st[:-1]:
+        ok = ok and s % 8 == 0
+    return x if ok else x.contiguous()
+
+
+def _bf16_rows(x):
+    """_rows of x in bf16."""
+    if x.dtype != torch.bfloat16:
+        x = x.to(torch.bfloat16)
+    return _rows(x)
 
 
 def kbar(idx_k, head_cls, block_size, cu_seqlens=None, seq_lens=None, nblk_cap=None,
@@ -1104,7 +1117,7 @@ def decode_step_fused(q, k, v, idx_q, idx_k, head_cls, kbar_cache, block_size, l
                       idx_scale, floor, sigma, K, topm, scale, seq_lens=None, block_table=None,
                       page_size=None, cand=None, width=None, out_dtype=torch.float32,
                       return_lse=False, q_pos=None, workspace=None, return_scores=False,
-                      no_alloc=False, kbar_table=None, bounds=None):
+                      no_alloc=False, kbar_table=None, bounds=None, return_routing=True):
     """decode_route followed by attn_decode of its routing, in two launches: the window
     part of the attention runs beside the router.  Same arguments and results as those
     two calls (q [B,H,D] or [B,H,1,D]; out [B,H,D]); returns (out, (idx, bias, valid))
@@ -1115,6 +1128,10 @@ def decode_step_fused(q, k, v, idx_q, idx_k, head_cls, kbar_cache, block_size, l
     workspace: a caller's buffer instead of the cached one; zero-filled before its first
     step and passed whole on every step (the routing words at its end start at zero,
     and each step leaves them zero).
+    return_routing=False (without return_lse, return_scores, no_alloc): out alone; the routing
+    shares one allocation.
+    The host's share of a small step is more than the GPU's (34 us against 16 us for one
+    sequence of 389 tokens), so tensors that need no conversion skip the conversion calls.
     A wide entmax (topm <= 0 or > 16) routes through _decode_route_wide and attends
     with attn_decode (three launches instead of two)."""
     _need_gpu(q, k, v, idx_q, idx_k, kbar_cache)
@@ -1133,23 +1150,23 @@ def decode_step_fused(q, k, v, idx_q, idx_k, head_cls, kbar_cache, block_size, l
                           block_table=block_table, page_size=page_size, out_dtype=out_dtype,
                           return_lse=True)
         out, lse = res
+        if not (return_routing or return_lse or return_scores):
+            return out[:, :, None] if squeeze else out
         return _step_result(out, lse if return_lse else None, idx[:, 0], bias[:, 0], valid[:, 0],
                             z, squeeze, return_lse, return_scores)
     lib = _lib.load()
     squeeze = q.dim() == 4
     if squeeze:
         q = q[:, :, 0]
-    q = _rows(q.to(torch.bfloat16))
-    k = _rows(k.to(torch.bfloat16))
-    v = _rows(v.to(torch.bfloat16))
-    if idx_q.dim() == 3:
-        idx_q = idx_q[:, 0]
-    idx_q = idx_q.float().contiguous()
-    idx_k = idx_k.float()
+    q, k, v = _bf16_rows(q), _bf16_rows(k), _bf16_rows(v)
+    if idx_q.dtype != torch.float32 or not idx_q.is_contiguous():
+        idx_q = (idx_q[:, 0] if idx_q.dim() == 3 else idx_q).float().contiguous()
+    if idx_k.dtype != torch.float32:
+        idx_k = idx_k.float()
     if idx_k.stride(-1) != 1:
         idx_k = idx_k.contiguous()
     B, H, D = q.shape
-    d = idx_q.shape[1]
+    d = idx_q.shape[-1]
     nblk_cap, kb_sb, kbt, kb_ts, bnd = _kbar_layout(kbar_cache, kbar_table, bounds)
     if block_table is not None:
         bt = _i32(block_table)
@@ -1169,15 +1186,27 @@ def decode_step_fused(q, k, v, idx_q, idx_k, head_cls, kbar_cache, block_size, l
     if seq_lens is None and width is None:
         Kw = max(1, min(int(K), max(1, min(int(topm), (S + block_size - 1) // block_size))))
     dev = q.device
-    idx = torch.empty(B, Kw, dtype=torch.int32, device=dev)
-    bias = torch.empty(B, Kw, dtype=torch.float32, device=dev)
-    valid = torch.empty(B, Kw, dtype=torch.uint8, device=dev)
-    z = torch.empty(B, nblk_cap, dtype=torch.float32, device=dev)
     out = torch.empty(B, H, D, dtype=out_dtype, device=dev)
-    lse = torch.empty(B, H, dtype=torch.float32, device=dev) if return_lse else None
+    bare = not (return_routing or return_lse or return_scores or no_alloc)
+    if bare:
+        # idx, bias, z and valid in one buffer, 16-byte aligned pieces
+        n, nz = (B * Kw * 4 + 15) // 16 * 16, (B * nblk_cap * 4 + 15) // 16 * 16
+        buf = torch.empty(3 * n + nz, dtype=torch.uint8, device=dev)
+        p_idx = buf.data_ptr()
+        p_bias, p_z, p_valid = p_idx + n, p_idx + 2 * n, p_idx + 2 * n + nz
+        idx = bias = valid = z = lse = None
+    else:
+        idx = torch.empty(B, Kw, dtype=torch.int32, device=dev)
+        bias = torch.empty(B, Kw, dtype=torch.float32, device=dev)
+        valid = torch.empty(B, Kw, dtype=torch.uint8, device=dev)
+        z = torch.empty(B, nblk_cap, dtype=torch.float32, device=dev)
+        lse = torch.empty(B, H, dtype=torch.float32, device=dev) if return_lse else None
+        p_idx, p_bias, p_valid, p_z = (t.data_ptr() for t in (idx, bias, valid, z))
     lens = _i32(seq_lens)
     c2 = None if cand is None else _u8(cand.reshape(B, -1))
-    hc = head_cls.float().contiguous()
+    hc = head_cls
+    if hc.dtype != torch.float32 or not hc.is_contiguous():
+        hc = hc.float().contiguous()
     lw = int(local_blocks) * int(block_size)
     qp = None if q_pos is None else _i32(q_pos.reshape(B))
     if no_alloc:
@@ -1195,30 +1224,39 @@ def decode_step_fused(q, k, v, idx_q, idx_k, head_cls, kbar_cache, block_size, l
             B, H, D, int(block_size), lw, float(scale), _stream())
         _lib.check(st_, "dash_decode_step_noalloc")
         return _step_result(out, lse, idx, bias, valid, z, squeeze, return_lse, return_scores)
-    ws_bytes = ctypes.c_int64(0)
-    _lib.check(lib.dash_decode_step_workspace_size(B, H, D, int(block_size), lw, ws_bytes),
-               "workspace")
+    ws_bytes = _step_workspace_size(B, H, D, int(block_size), lw)
     if workspace is None:
-        ws = _step_workspace(ws_bytes.value, dev)
+        ws = _step_workspace(ws_bytes, dev)
     else:
         ws = workspace
-        if ws.numel() * ws.element_size() < ws_bytes.value:
+        if ws.numel() * ws.element_size() < ws_bytes:
             raise ValueError("decode step workspace too small")
     st_ = lib.dash_decode_step(
-        _ptr(idx_q), idx_q.stride(0), _ptr(idx_k), isb, ist, isp, _ptr(bt), bt_stride,
-        int(page_size or 0), _ptr(lens), _ptr(qp), S, _ptr(hc), 1, _ptr(kbar_cache),
+        idx_q.data_ptr(), idx_q.stride(0), idx_k.data_ptr(), isb, ist, isp, _ptr(bt), bt_stride,
+        int(page_size or 0), _ptr(lens), _ptr(qp), S, hc.data_ptr(), 1, kbar_cache.data_ptr(),
         kb_sb, nblk_cap, _ptr(kbt), kb_ts, _ptr(bnd), _ptr(c2),
         0 if c2 is None else c2.stride(0), d, int(local_blocks),
-        float(idx_scale), float(floor), float(sigma), int(K), int(topm), Kw, _ptr(idx),
-        _ptr(bias), _ptr(valid), _ptr(z), z.stride(0),
-        _ptr(q), q.stride(0), q.stride(1),
-        _ptr(k), k_sb, k_sh, k_st, k_sp, _ptr(v), v_sb, v_sh, v_st, v_sp,
-        _ptr(out), int(out_dtype == torch.bfloat16), out.stride(0), out.stride(1),
+        float(idx_scale), float(floor), float(sigma), int(K), int(topm), Kw, p_idx,
+        p_bias, p_valid, p_z, nblk_cap,
+        q.data_ptr(), q.stride(0), q.stride(1),
+        k.data_ptr(), k_sb, k_sh, k_st, k_sp, v.data_ptr(), v_sb, v_sh, v_st, v_sp,
+        out.data_ptr(), int(out_dtype == torch.bfloat16), H * D, D,
         _ptr(lse), 0 if lse is None else lse.stride(0), 1,
-        B, H, D, int(block_size), lw, float(scale), _ptr(ws), ws.numel() * ws.element_size(),
+        B, H, D, int(block_size), lw, float(scale), ws.data_ptr(), ws.numel() * ws.element_size(),
         _stream())
-    _lib.check(st_, "dash_decode_step")
+    if st_ != 0:
+        _lib.check(st_, "dash_decode_step")
+    if bare:
+        return out[:, :, None] if squeeze else out
     return _step_result(out, lse, idx, bias, valid, z, squeeze, return_lse, return_scores)
+
+
+@functools.lru_cache(maxsize=256)
+def _step_workspace_size(B, H, D, block_size, lw):
+    nbytes = ctypes.c_int64(0)
+    _lib.check(_lib.load().dash_decode_step_workspace_size(B, H, D, block_size, lw, nbytes),
+               "workspace")
+    return nbytes.value
 
 
 _STEP_WORKSPACES = {}
@@ -1229,7 +1267,7 @@ def _step_workspace(nbytes, device):
     routing words at its end must start at zero; every step leaves them zero), and
     always passed whole, so those words stay in one place.  Calls that share it are
     ordered on the current stream."""
-    k = str(device)
+    k = device
     buf = _STEP_WORKSPACES.get(k)
     if buf is None or buf.numel() * 4 < nbytes:
         if buf is not None:

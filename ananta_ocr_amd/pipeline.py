@@ -218,15 +218,16 @@ def decode_step(state, q, k, v, idx_q, idx_k, head_cls, block_size, local_blocks
         npw = (local_blocks * block_size + block_size - 1 + 31) // 32
         fused = nsplit is None and D == 128 and slots <= 16 and npw + slots <= 64
     if fused:
-        out, (idx, bias, valid), z = ops.decode_step_fused(
+        res = ops.decode_step_fused(
             q, k, v, idx_q, idx_k, head_cls, state.kbar, block_size, local_blocks, idx_scale,
             floor, sigma, K, topm, scale, seq_lens=seq_lens, block_table=block_table,
             page_size=page_size, cand=block_cand, width=width, out_dtype=out_dtype,
-            return_scores=True, **kbx)
-        if return_routing:
-            res = (out, (idx, bias, valid.bool()))
-            return res + (z,) if return_scores else res
-        return out
+            return_scores=return_routing, return_routing=return_routing, **kbx)
+        if not return_routing:
+            return res
+        out, (idx, bias, valid), z = res
+        res = (out, (idx, bias, valid.bool()))
+        return res + (z,) if return_scores else res
     idx, bias, valid, z = ops.decode_route(idx_q, idx_k, head_cls, state.kbar, block_size,
                                            local_blocks, idx_scale, floor, sigma, K, topm,
                                            seq_lens=seq_lens, block_table=block_table,
