@@ -1757,9 +1757,10 @@ struct BwdLayout {
   int nstage, part_steps, item_cap, slot_cap;
 };
 // Steps of a part of a key-major stage, at least; a stage's window steps count double where
-// they are more, so that the stages in parts are those of many pairs.  A third of a CU's even
-// share of the pairs' steps, 24 to 128: the heaviest stages start first, so that such parts
-// still end together, and a part's start and its 64 KB of sums cost about two steps.
+// they are more, so that the stages in parts are those of many pairs.  A fifth of a CU's even
+// share of the pairs' steps (two work-groups run on it), 24 to 128: the heaviest stages start
+// first, so that such parts still end together, and a part's start and its 64 KB of sums
+// cost about two steps.
 constexpr int kBwMinSteps = 24, kBwMaxSteps = 128;
 
 inline BwdLayout bwd_layout(int B, int H, int S_max, int64_t rows, int K, int D, int nblk_cap,
@@ -1775,7 +1776,7 @@ inline BwdLayout bwd_layout(int B, int H, int S_max, int64_t rows, int K, int D,
   L.nstage = (int)(((int64_t)nblk_cap * bs + kBwIT - 1) / kBwIT);
   // stages that take a block's pairs
   const int64_t per = bs <= kBwIT ? 1 : bs % kBwIT == 0 ? nsub : nsub + 1;
-  const int64_t est = H * (per * rows * K / kBwIT + rows / kBwIT + B) / (256 * 3);
+  const int64_t est = H * (per * rows * K / kBwIT + rows / kBwIT + B) / (256 * 5);
   L.part_steps = (int)std::min<int64_t>(std::max<int64_t>(est, kBwMinSteps), kBwMaxSteps);
   // a stage in parts of X steps has more than X / 2 steps of pairs (r), so at most
   // (r + X / 2) / X + 1 <= 4 r / X parts
@@ -2070,7 +2071,7 @@ extern "C" int dash_attn_prefill_backward(
     hipLaunchKernelGGL(prefill_scatter_kernel, dim3(p.ntiles, B), dim3(kPfTQ), 0, st, p);
   }
   hipLaunchKernelGGL(bwd_items_kernel, dim3(B), dim3(256), 0, st, a);
-  hipLaunchKernelGGL(bwd_kv_kernel, dim3(stream_stage_grid(B * H, a.item_cap)), dim3(512), 0, st, a);
+  hipLaunchKernelGGL(bwd_kv_kernel, dim3(stream_stage_grid(B * H, a.item_cap)), dim3(256), 0, st, a);
   if (K > 0)
     hipLaunchKernelGGL(bwd_sum_kernel, dim3(4 * a.nstage, H, B), dim3(256), 0, st, a);
   hipLaunchKernelGGL(bwd_q_kernel, dim3(p.ntiles * H * B), dim3(256), 0, st, a);

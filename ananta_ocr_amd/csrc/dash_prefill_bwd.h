@@ -15,18 +15,13 @@
 //   * key-major kernel, one work-group per (64-key stage, head, sequence): the
 //     stage's K and V stay in LDS while 64 queries at a time stream through it --
 //     first the window band (every query whose window reaches the stage), then
-//     the routed pairs of the stage's blocks, gathered.  Per 32-query chunk and
-//     32-key half, two wavefronts (one per half of the head dims), each computing
-//     S = Q K^T and dP = dO V^T on the matrix cores (lane = key), P and dS in
-//     registers, and its dims of dV^T += dO^T P and dK^T += Q^T dS, the transposed
-//     operands read by ds_read_tr16_b64.  dK
-//     and dV are complete when the work-group ends (no atomics).  For routed
-//     pairs it also writes dQ^T = K^T dS^T (dS through LDS, read transposed) and
-//     the row sums of dS as fp32 partials per (head, pair).  The steps are
-//     software-pipelined: a step's query rows load into the other of two LDS
-//     buffers while the previous step computes, their row numbers and per-query
-//     values one step earlier still, and a routed step's partials are stored
-//     whole rows at a time at the start of the next step;
+//     the routed pairs of the stage's blocks, gathered.  One wavefront per 32-query
+//     chunk and 32-key half computes S = Q K^T and dP = dO V^T on the matrix cores
+//     (lane = key), P and dS in registers, dV^T += dO^T P and dK^T += Q^T dS, the
+//     transposed operands read by ds_read_tr16_b64.  dK and dV are complete when the
+//     work-group ends (no atomics), or added over the parts of a heavy stage.  For
+//     routed pairs it also writes dQ^T = K^T dS^T (dS through LDS, read transposed) and
+//     the row sums of dS as partials per (head, pair);
 //   * query-major kernel, one work-group per (128-query tile, head, sequence),
 //     lane = query: dQ^T += K^T dS^T over the window band (S^T, dP^T recomputed),
 //     plus the query's routed partials, times the scale;
@@ -241,32 +236,37 @@ __device__ __forceinline__ TrOff bw_tr_lane_off(int qbase, int lane) {
   return {lo, hi};
 }
 
-// Loads rows of a 64-row, bw_swz-swizzled stage by 8 wavefronts: wavefront wv,
-// lane l fills slot l % 16 of rows 32 u + r0 (r0 = 4 wv + l / 16, u < 2) from the
-// row pointer rowp(r).
-template <typename RowPtr>
-__device__ __forceinline__ void stage_rows8(bf16* sX, int wv, int lane, RowPtr rowp) {
+// stage_rows with the lane's four row numbers given (row 16 u + r0 of the stage); row
+// numbers are >= 0 and the row stride is below 2^32 elements.
+__device__ __forceinline__ void stage_rows4r(bf16* sX, int wv, int lane, const bf16* xb, int64_t x_st,
+                                             int4 rw) {
   const int r0 = 4 * wv + (lane >> 4), slot = lane & 15;
+  const int rr[4] = {rw.x, rw.y, rw.z, rw.w};
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int r = 32 * u + r0;
-    __builtin_amdgcn_global_load_lds((const void*)(rowp(r) + (slot ^ bw_swz(r0 & 15)) * 8),
-                                     (__attribute__((address_space(3))) void*)(sX + (32 * u + 4 * wv) * 128),
-                                     16, 0, 0);
-  }
-}
-// The same with the lane's two row numbers given (rw.x: row r0, rw.y: row 32 + r0);
-// row numbers are >= 0 and the row stride is below 2^32 elements.
-__device__ __forceinline__ void stage_rows8r(bf16* sX, int wv, int lane, const bf16* xb, int64_t x_st,
-                                             int2 rw) {
-  const int r0 = 4 * wv + (lane >> 4), slot = lane & 15;
-  const int rr[2] = {rw.x, rw.y};
-#pragma unroll
-  for (int u = 0; u < 2; ++u)
+  for (int u = 0; u < 4; ++u)
     __builtin_amdgcn_global_load_lds((const void*)(xb + (uint64_t)(uint32_t)rr[u] * (uint32_t)x_st +
-                                                   (slot ^ bw_swz(r0 & 15)) * 8),
-                                     (__attribute__((address_space(3))) void*)(sX + (32 * u + 4 * wv) * 128),
+                                                   (slot ^ bw_swz(r0)) * 8),
+                                     (__attribute__((address_space(3))) void*)(sX + (16 * u + 4 * wv) * 128),
                                      16, 0, 0);
+}
+
+// Sums over the 32 lanes of each wavefront half of 16 values per lane: afterwards lanes
+// with (lane / 16) % 2 == p hold in v[0..7] the totals of values 8 p + 0..7.
+__device__ __forceinline__ void half_sums16(float (&v)[16]) {
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[k]), __float_as_uint(v[k + 8]), false, false);
+    v[k] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    float x = v[k];
+    x += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x128, 0xf, 0xf, false));
+    x += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x124, 0xf, 0xf, false));
+    x += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x122, 0xf, 0xf, false));
+    x += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x121, 0xf, 0xf, false));
+    v[k] = x;
+  }
 }
 
 // The steps of a key-major stage: n_win 64-query steps of the window band, then the routed
@@ -336,37 +336,34 @@ __global__ __launch_bounds__(256) void bwd_items_kernel(BwdArgs a) {
   if (tid == 0) a.n_items[b] = min(item0, a.item_cap);
 }
 
-// Key-major kernel, eight wavefronts: wavefront (kh, qc, dh) = (wv % 2, wv / 2 % 2,
-// wv / 4) owns keys 32 kh .. + 31 of the stage, queries 32 qc .. + 31 of a step and
-// head dims 64 dh .. + 63 of dK and dV, so that two wavefronts fit on a SIMD.  Per
-// step both wavefronts of a (kh, qc) pair compute S, P, dP and dS (the products are
-// cheap here; an exchange through LDS cost a barrier), and each adds its dims'
-// share of dV^T += dO^T P and dK^T += Q^T dS.  Routed steps: dQ^T = K^T dS^T
-// for the step's 64 queries x 128 dims, one 32 x 32 tile per wavefront (dims
-// 32 (2 dh + kh) ..), and the bias-gradient row sums.
-// Software pipeline over the steps: step s computes on the query rows in buffer
-// s % 2 with the per-query values in sM[s % 2]; meanwhile the rows of step s + 1
-// load into the other buffer (row numbers from sRow[(s + 1) % 2]), and wavefront 0
-// loads the values of step s + 1 and the pair ids of step s + 2, which it stores
-// after the products (sM[(s + 1) % 2], sRow[s % 2]).  A routed step's dQ^T partials
-// wait in LDS and are stored at the start of the next step, so that the wait that
-// ends a step does not wait for stores just issued.  One wait and one barrier end
-// each step.
-__global__ __launch_bounds__(512, 1) void bwd_kv_kernel(BwdArgs a) {
+// Key-major kernel, four wavefronts, two work-groups per CU: wavefront (kh, qc) = (wv % 2,
+// wv / 2) owns keys 32 kh .. + 31 of the stage and queries 32 qc .. + 31 of a step.  It forms
+// its 32 x 32 tile of S, dP, P and dS once and adds it to its keys' dV^T += dO^T P and dK^T +=
+// Q^T dS for all 128 head dims (128 accumulator registers).  Routed steps: dQ^T = K^T dS^T
+// for the step's 64 queries x 128 dims, two 32 x 32 tiles per wavefront (dims 64 kh ..), and
+// the bias-gradient row sums.
+// A step waits for its rows (one barrier), computes, and after a second barrier (every
+// wavefront has read the rows; dS is in LDS) loads the next step's rows over them, beside
+// the dQ products; the other work-group of the CU computes while this one waits.  Row
+// numbers and per-query values are loaded one to two steps ahead by wavefront 0.  dQ^T
+// partials stay in registers until the next step has begun, so that its wait for the rows
+// does not wait for stores just issued.
+// One work-group of eight wavefronts per CU with two row buffers, in which two wavefronts
+// formed each tile of S and dP (one per half of the head dims), took 1,630 us against 1,160
+// for 27,300 tokens, 10 heads, window 1,024, 16 routed blocks of 64, and 988 against 745 for
+// window 128, 12 of 32.  What bounds it: the waits for rows and barriers (46 % of the
+// wavefronts' time), then vector and matrix instructions (40 % and 25 % of the cycles).
+__global__ __launch_bounds__(256, 2) void bwd_kv_kernel(BwdArgs a) {
   constexpr int D = 128;
   __shared__ __attribute__((aligned(16))) bf16 sK[kBwIT * D];
   __shared__ __attribute__((aligned(16))) bf16 sV[kBwIT * D];
-  __shared__ __attribute__((aligned(16))) bf16 sQ0[kBwIT * D];
-  __shared__ __attribute__((aligned(16))) bf16 sQ1[kBwIT * D];
-  __shared__ __attribute__((aligned(16))) bf16 sO0[kBwIT * D];   // dO rows
-  __shared__ __attribute__((aligned(16))) bf16 sO1[kBwIT * D];
+  __shared__ __attribute__((aligned(16))) bf16 sQ[kBwIT * D];
+  __shared__ __attribute__((aligned(16))) bf16 sO[kBwIT * D];      // dO rows
   __shared__ __attribute__((aligned(16))) bf16 sDS[2][kBwIT][36];  // dS [qc][key][query]
   __shared__ __attribute__((aligned(16))) KvMeta sM[2];
-  // row numbers of a step for the loads: query slot q at [q % 32][q / 32]
-  __shared__ __attribute__((aligned(16))) int sRow[2][32][2];
-  __shared__ float sDb[2][kBwIT];
-  // per wavefront 4 KB: the dQ^T staging of a routed step until the start of the next
-  __shared__ __attribute__((aligned(16))) float sX[8][1024];
+  // row numbers of a step for the loads: query slot q at [q % 16][q / 16]
+  __shared__ __attribute__((aligned(16))) int sRow[2][16][4];
+  __shared__ __attribute__((aligned(16))) float sDb[2][kBwIT];
 
   const PrefillArgs& p = a.p;
   // Stages in order per (sequence, head) stream, each stream's stages on one XCD
@@ -380,13 +377,19 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_kernel(BwdArgs a) {
   if (!stream_stage_item((int)blockIdx.x, p.B * p.H, a.item_cap, bh, item)) return;
   const int h = bh % p.H, b = bh / p.H;
   if (item >= a.n_items[b]) return;
-  const int4 it = a.items[(int64_t)b * a.item_cap + item];
+  // uniform values loaded through vector memory are made scalar
+  auto uni = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+  int4 it = a.items[(int64_t)b * a.item_cap + item];
+  it = make_int4(uni(it.x), uni(it.y), uni(it.z), uni(it.w));
   const int nparts = it.z;
-  const int len = seq_len(p, b);
+  const int len = uni(seq_len(p, b));
   const int j0 = it.x * kBwIT;
   const int sub = (j0 % p.bs) / kBwIT;
-  const int tid = threadIdx.x, lane = wave_lane(), wv = tid / kWave;
-  const int kh = wv & 1, qc = (wv >> 1) & 1, dh = wv >> 2, hl = lane >> 5, n = lane & 31;
+  // the lane's numbers pass through an empty asm each step, so that what follows from them
+  // is formed there instead of being kept in registers (or spilled) across the steps
+  int tid = threadIdx.x, lane = wave_lane(), hl = lane >> 5, n = lane & 31;
+  const int wv = uni(tid / kWave);
+  const int kh = wv & 1, qc = wv >> 1;
   const int64_t r0 = row0(p, b);
   const float c2 = a.scale * 1.4426950408889634f;
   const float log2e = 1.4426950408889634f;
@@ -395,17 +398,17 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_kernel(BwdArgs a) {
   const bf16* vb = seq_base(p.v, p.cu, b, p.v_sb, p.v_st) + (int64_t)h * p.v_sh;
   const bf16* qb = seq_base(p.q, p.cu, b, p.q_sb, p.q_st) + (int64_t)h * p.q_sh;
   const bf16* ob = seq_base(a.dout, p.cu, b, a.do_sb, a.do_st) + (int64_t)h * a.do_sh;
-  stage_rows8(sK, wv, lane, [&](int r) { return kb + (int64_t)min(j0 + r, len - 1) * p.k_st; });
-  stage_rows8(sV, wv, lane, [&](int r) { return vb + (int64_t)min(j0 + r, len - 1) * p.v_st; });
+  stage_rows(sK, wv, lane, [&](int r) { return kb + (int64_t)min(j0 + r, len - 1) * p.k_st; });
+  stage_rows(sV, wv, lane, [&](int r) { return vb + (int64_t)min(j0 + r, len - 1) * p.v_st; });
 
   const int LW = p.lw, bs = p.bs;
   const int c_first = j0 / bs;
   const KvSteps ks_ = kv_steps(p, b, len, j0);
-  const int n_win = ks_.n_win, rs0 = ks_.rs0;
-  const int np0 = ks_.np0, np1 = ks_.np1, ch00 = ks_.ch00, ch01 = ks_.ch01;
+  const int n_win = uni(ks_.n_win), rs0 = uni(ks_.rs0);
+  const int np0 = uni(ks_.np0), np1 = uni(ks_.np1), ch00 = uni(ks_.ch00), ch01 = uni(ks_.ch01);
   // this part's steps [s_first, n_steps)
-  const int s_first = (int)((int64_t)ks_.n * it.y / nparts);
-  const int n_steps = (int)((int64_t)ks_.n * (it.y + 1) / nparts);
+  const int s_first = uni((int)((int64_t)ks_.n * it.y / nparts));
+  const int n_steps = uni((int)((int64_t)ks_.n * (it.y + 1) / nparts));
 
   auto pair_of = [&](int u) -> int {
     const int v = u - n_win;
@@ -455,18 +458,14 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_kernel(BwdArgs a) {
     M.pos[tid] = m.ok ? m.pos : -1;
   };
 
-  floatx16 acc_dk[2], acc_dv[2];           // dims 64 dh + 32 t ..
+  floatx16 acc_dk[4], acc_dv[4];           // dims 32 t ..
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < 4; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) { acc_dk[t][r] = 0.f; acc_dv[t][r] = 0.f; }
 
-  const uint32_t kl0 = bw_k_lane_off(n, hl);
-  const TrOff tq0 = bw_tr_lane_off(32 * qc, lane), tk0 = bw_tr_lane_off(0, lane);
-  const int key = j0 + 32 * kh + n;
   const int kst = 32 * kh, qst = 32 * qc;
-  const int dtq = 2 * dh + kh;             // this wavefront's dQ dim tile
-  float* const xs = sX[wv];                // own staging area
+  int rl = 4 * wv + (lane >> 4);           // this lane's rows 16 u + rl of a step
 
   int pid_next = -1;
   if (n_steps > s_first) {
@@ -474,72 +473,59 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_kernel(BwdArgs a) {
       const int pid0 = s_first < n_win ? -1 : pair_of(s_first);
       pid_next = s_first + 1 < n_steps && s_first + 1 >= n_win ? pair_of(s_first + 1) : -1;
       meta_store(s_first, meta_load(s_first, pid0), sM[0]);
-      sRow[0][tid & 31][tid >> 5] = row_of(s_first, pid0);
-      if (s_first + 1 < n_steps) sRow[1][tid & 31][tid >> 5] = row_of(s_first + 1, pid_next);
+      sRow[0][tid & 15][tid >> 4] = row_of(s_first, pid0);
+      if (s_first + 1 < n_steps) sRow[1][tid & 15][tid >> 4] = row_of(s_first + 1, pid_next);
     }
     __syncthreads();
-    const int2 rw = *(const int2*)&sRow[0][4 * wv + (lane >> 4)][0];
-    stage_rows8r(sQ0, wv, lane, qb, p.q_st, rw);
-    stage_rows8r(sO0, wv, lane, ob, a.do_st, rw);
+    const int4 rw = *(const int4*)&sRow[0][rl][0];
+    stage_rows4r(sQ, wv, lane, qb, p.q_st, rw);
+    stage_rows4r(sO, wv, lane, ob, a.do_st, rw);
   }
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
 
-  // dQ^T partials of a routed step wait in the wavefront's area (query row r at 32
-  // halves, 8-byte chunk c in slot c ^ (r % 8), the row's scale at float 512 + r) and
-  // are stored at the start of the next step, 8 lanes per 64-byte row piece.
-  bool pend = false;
-  int64_t pend_pi = -1;
-  float pend_db = 0.f;
-  auto store_pending = [&](int par) {
-    if (pend) {
-      const int c = lane & 7;
-      const _Float16* const xh = (const _Float16*)xs;
+  // A routed step's dQ^T partials: dims 64 kh + 32 t + 8 g + 4 hl + j of query qst + n, the
+  // 32 fp16 values contiguous in the partial row, with the pieces' scales
+  f16x8 pend_q[2][2];
+  float pend_sc[2], pend_db = 0.f;
+  int pend_pos = -1;
+  auto store_pending = [&]() {
+    if (pend_pos >= 0) {
+      const int64_t pi = ((int64_t)h * p.ppos + pend_pos) * a.nsub + sub;
+      _Float16* const o = a.part_dq + pi * D + 64 * hl + 32 * kh;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = 8 * i + (lane >> 3);
-        const int pos = sM[par].pos[qst + r];
-        const f16x4 v = *(const f16x4*)(xh + r * 32 + ((c ^ (r & 7)) << 2));
-        if (pos >= 0) {
-          const int64_t pi = ((int64_t)h * p.ppos + pos) * a.nsub + sub;
-          *(f16x4*)(a.part_dq + pi * D + (c & 1) * 64 + 16 * dtq + 4 * (c >> 1)) = v;
-          if (c == 0) a.part_dqs[pi * 4 + dtq] = xs[512 + r];
-        }
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) *(f16x8*)(o + 16 * t + 8 * c) = pend_q[t][c];
+      if (hl == 0) {
+        *(float2*)(a.part_dqs + pi * 4 + 2 * kh) = make_float2(pend_sc[0], pend_sc[1]);
+        if (kh == 0) a.part_db[pi] = pend_db;
       }
-      if (kh == 0 && dh == 0 && hl == 0 && pend_pi >= 0) a.part_db[pend_pi] = pend_db;
     }
-    pend = false;
+    pend_pos = -1;
   };
 
-  auto step = [&](int s, auto par_tag) {
-    constexpr int P = decltype(par_tag)::value;
-    const bf16* const sQ = P == 0 ? sQ0 : sQ1;
-    const bf16* const sO = P == 0 ? sO0 : sO1;
-    bf16* const sQn = P == 0 ? sQ1 : sQ0;
-    bf16* const sOn = P == 0 ? sO1 : sO0;
+  for (int s = s_first; s < n_steps; ++s) {
+    const int P = (s - s_first) & 1;
     const KvMeta& M = sM[P];
     const bool routed = s >= n_win;
-    store_pending(P ^ 1);
-    if (s + 1 < n_steps) {
-      const int2 rw = *(const int2*)&sRow[P ^ 1][4 * wv + (lane >> 4)][0];
-      stage_rows8r(sQn, wv, lane, qb, p.q_st, rw);
-      stage_rows8r(sOn, wv, lane, ob, a.do_st, rw);
-    }
-    uint32_t kl = kl0;
-    TrOff tq = tq0, tk = tk0;
-    asm volatile("" : "+v"(kl), "+v"(tq.lo), "+v"(tq.hi), "+v"(tk.lo), "+v"(tk.hi));
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();                       // the step's rows and values are there
+    store_pending();
+    asm volatile("" : "+v"(tid));
+    lane = tid & (kWave - 1);
+    hl = lane >> 5;
+    n = lane & 31;
+    rl = 4 * wv + (lane >> 4);
+    const int key = j0 + 32 * kh + n;
+    const uint32_t kl = bw_k_lane_off(n, hl);
+    const TrOff tq = bw_tr_lane_off(32 * qc, lane);
     KvMetaLoad ml = {};
     int pid2 = -1;
     if (wv == 0) {
       if (s + 1 < n_steps) ml = meta_load(s + 1, pid_next);
       if (s + 2 < n_steps && s + 2 >= n_win) pid2 = pair_of(s + 2);
     }
-
     // S and dP of the (kh, qc) tile, lane = key, rows = queries 8 g + 4 hl + j of the
-    // chunk.  Both wavefronts of a dim pair compute both (the matrix cores have room;
-    // no exchange and no barrier between them).  The next k-step's four operand reads
-    // are issued before the current k-step's two products, fenced by scheduling
-    // barriers (left to itself the scheduler reads just before each product).
+    // chunk; the next k-step's operand reads are issued before the current products
     floatx16 xs_, xd_;
 #pragma unroll
     for (int r = 0; r < 16; ++r) { xs_[r] = 0.f; xd_[r] = 0.f; }
@@ -558,17 +544,18 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_kernel(BwdArgs a) {
         __builtin_amdgcn_sched_barrier(0);
         xs_ = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f0[0], f0[1], xs_, 0, 0, 0);
         xd_ = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f0[2], f0[3], xd_, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" : "+v"(xs_), "+v"(xd_));     // the products stay before the next reads
         if (kk + 2 < D / 16) rd(kk + 2, f0);
         __builtin_amdgcn_sched_barrier(0);
         xs_ = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f1[0], f1[1], xs_, 0, 0, 0);
         xd_ = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f1[2], f1[3], xd_, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" : "+v"(xs_), "+v"(xd_));
       }
     }
-    float pr[16], ds[16];
+    // P into xs_, dS into xd_
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
+      __builtin_amdgcn_sched_barrier(0);
       const int q0 = qst + 8 * g + 4 * hl;
       const float4 l2 = *(const float4*)&M.l2[q0];
       const float4 b2 = *(const float4*)&M.b2[q0];
@@ -585,74 +572,63 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_kernel(BwdArgs a) {
         const int r = 4 * g + j;
         const float e = fast_exp2(fmaf(xs_[r], c2, b2a[j] - l2a[j]));
         const bool vis = (key >= loa[j]) & (key <= hia[j]);
-        pr[r] = vis ? e : 0.f;
-        ds[r] = pr[r] * (xd_[r] - dea[j]);
+        xs_[r] = vis ? e : 0.f;
+        xd_[r] = xs_[r] * (xd_[r] - dea[j]);
       }
     }
-    // this wavefront's dims of dV^T += dO^T P and dK^T += Q^T dS (operand reads
-    // issued together, as above)
-    floatx16 pf, df;
+    // dV^T += dO^T P and dK^T += Q^T dS
 #pragma unroll
-    for (int r = 0; r < 16; ++r) { pf[r] = pr[r]; df[r] = ds[r]; }
-    {
-      bf16x8 fo[2][2], fq[2][2];
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          fo[ks][t] = tr_frag_at(sO, tq, ks, 2 * dh + t);
-          fq[ks][t] = tr_frag_at(sQ, tq, ks, 2 * dh + t);
-        }
+    for (int ks = 0; ks < 2; ++ks) {
+      const bf16x8 pb = acc_bop(xs_, ks);
+      const bf16x8 db = acc_bop(xd_, ks);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        const bf16x8 pb = acc_bop(pf, ks);
-        const bf16x8 db = acc_bop(df, ks);
+      for (int t = 0; t < 4; ++t)
+        acc_dv[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag_at(sO, tq, ks, t), pb, acc_dv[t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          acc_dv[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fo[ks][t], pb, acc_dv[t], 0, 0, 0);
-          acc_dk[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fq[ks][t], db, acc_dk[t], 0, 0, 0);
-        }
-      }
+      for (int t = 0; t < 4; ++t)
+        acc_dk[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag_at(sQ, tq, ks, t), db, acc_dk[t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
     if (routed) {
-      if (dh == 0) {
-        // dS through LDS (sDS[qc][key][query]) and its row sums over this
-        // wavefront's 32 keys
+      // dS through LDS (sDS[qc][key][query]), and its row sums over this wavefront's 32
+      // keys in fp32
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          bf16x4 w;
+      for (int g = 0; g < 4; ++g) {
+        bf16x4 w;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) w[j] = (bf16)ds[4 * g + j];
-          *(bf16x4*)&sDS[qc][kst + n][8 * g + 4 * hl] = w;
-        }
-        // the row sums in fp32: ds through the wavefront's staging area (free between the
-        // previous step's partial stores and this step's staging) as [key][query], in the
-        // staging's swizzle, then lanes q and q + 32 add 16 keys each (16 shuffle-sums of
-        // 32 lanes cost more)
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          *(float4*)(xs + n * 32 + (((2 * g + hl) ^ (n & 7)) << 2)) =
-              make_float4(ds[4 * g], ds[4 * g + 1], ds[4 * g + 2], ds[4 * g + 3]);
-        wave_lds_sync();
-        {
-          const int q = lane & 31;
-          float sum = 0.f;
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int key = 16 * hl + i;
-            sum += xs[key * 32 + (((q >> 2) ^ (key & 7)) << 2) + (q & 3)];
-          }
-          sum += __shfl_xor(sum, 32, kWave);
-          if (hl == 0) sDb[kh][qst + q] = sum;
-        }
-        wave_lds_sync();
+        for (int j = 0; j < 4; ++j) w[j] = (bf16)xd_[4 * g + j];
+        *(bf16x4*)&sDS[qc][kst + n][8 * g + 4 * hl] = w;
       }
-      lds_barrier();
-      // dQ^T tile dtq = K^T dS^T over the stage's 64 keys for the chunk's 32 queries
-      floatx16 acc_q;
+      float v[16];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc_q[r] = 0.f;
+      for (int r = 0; r < 16; ++r) v[r] = xd_[r];
+      half_sums16(v);
+      if ((lane & 15) == 0) {
+        const int q0 = qst + 16 * ((lane >> 4) & 1) + 4 * hl;
+        *(float4*)&sDb[kh][q0] = make_float4(v[0], v[1], v[2], v[3]);
+        *(float4*)&sDb[kh][q0 + 8] = make_float4(v[4], v[5], v[6], v[7]);
+      }
+    }
+    if (wv == 0) {
+      if (s + 1 < n_steps) meta_store(s + 1, ml, sM[P ^ 1]);
+      if (s + 2 < n_steps) sRow[P][tid & 15][tid >> 4] = row_of(s + 2, pid2);
+      pid_next = pid2;
+    }
+    lds_barrier();                         // the rows are read, dS is written
+    if (s + 1 < n_steps) {
+      const int4 rw = *(const int4*)&sRow[P ^ 1][rl][0];
+      stage_rows4r(sQ, wv, lane, qb, p.q_st, rw);
+      stage_rows4r(sO, wv, lane, ob, a.do_st, rw);
+    }
+    if (routed) {
+      // dQ^T tiles 2 kh, 2 kh + 1 = K^T dS^T over the stage's 64 keys
+      asm volatile("" : "+v"(tid));
+      lane = tid & (kWave - 1);
+      hl = lane >> 5;
+      n = lane & 31;
+      const TrOff tk = bw_tr_lane_off(0, lane);
       const int tg = lane >> 4;
       const uint32_t dsa = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) bf16*)
           &sDS[qc][4 * (tg >> 1) + ((lane & 15) >> 2)][16 * (tg & 1) + 4 * (lane & 3)];
@@ -671,102 +647,90 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_kernel(BwdArgs a) {
             "=&v"(dst[6]), "=&v"(dst[7])
           : "v"(dsa)
           : "memory");
+      // one 32-dim piece at a time, in fp16 after scaling by 2^-e (lanes n and n + 32 hold
+      // its halves)
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        bf16x8 dsb;
+      for (int t = 0; t < 2; ++t) {
+        floatx16 acc_q;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) { dsb[e] = dst[2 * ks][e]; dsb[e + 4] = dst[2 * ks + 1][e]; }
-        acc_q = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag_at(sK, tk, ks, dtq), dsb, acc_q, 0, 0, 0);
+        for (int r = 0; r < 16; ++r) acc_q[r] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+          bf16x8 dsb;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { dsb[e] = dst[2 * ks][e]; dsb[e + 4] = dst[2 * ks + 1][e]; }
+          acc_q = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag_at(sK, tk, ks, 2 * kh + t), dsb, acc_q,
+                                                          0, 0, 0);
+        }
+        float mx = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, fabsf(acc_q[r]));
+        mx = xor32_max(mx);
+        const int ex = min(__builtin_amdgcn_frexp_expf(mx), 127);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) pend_q[t][r >> 3][r & 7] = (_Float16)ldexpf(acc_q[r], -ex);
+        pend_sc[t] = ldexpf(1.f, ex);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      // staged for the next step: dims 32 dtq + 8 g + 4 hl + j of query n, in fp16 after
-      // scaling by 2^-e (lanes n and n + 32 hold the two halves of the piece); the
-      // scale 2^e at xs[512 + n]
-      float mx = 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, fabsf(acc_q[r]));
-      mx = xor32_max(mx);
-      const int ex = min(__builtin_amdgcn_frexp_expf(mx), 127);
-      _Float16* const xh = (_Float16*)xs;
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        f16x4 hv;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) hv[j] = (_Float16)ldexpf(acc_q[4 * g + j], -ex);
-        *(f16x4*)(xh + n * 32 + (((2 * g + hl) ^ (n & 7)) << 2)) = hv;
-      }
-      if (hl == 0) xs[512 + n] = ldexpf(1.f, ex);
-      const int pos = M.pos[qst + n];
-      pend_pi = pos >= 0 ? ((int64_t)h * p.ppos + pos) * a.nsub + sub : -1;
+      pend_pos = M.pos[qst + n];
       pend_db = sDb[0][qst + n] + sDb[1][qst + n];
-      pend = true;
     }
-
-    if (wv == 0) {
-      if (s + 1 < n_steps) meta_store(s + 1, ml, sM[P ^ 1]);
-      if (s + 2 < n_steps) sRow[P][tid & 31][tid >> 5] = row_of(s + 2, pid2);
-      pid_next = pid2;
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-  };
-  int s = s_first;
-  for (; s + 1 < n_steps; s += 2) {
-    step(s, std::integral_constant<int, 0>{});
-    step(s + 1, std::integral_constant<int, 1>{});
   }
-  if (s < n_steps) step(s, std::integral_constant<int, 0>{});
-  store_pending((n_steps - s_first - 1) & 1);
+  store_pending();
 
-  // ---- dK and dV: the two query chunks' sums (16 KB per (kh, dh) pair) ----
-  const int ri = kh + 2 * dh;
-  float* const red = (float*)(ri == 0 ? sQ0 : ri == 1 ? sQ1 : ri == 2 ? sO0 : sO1);
+  // ---- dK and dV: the two query chunks' sums (32 KB per key half) ----
+  const int key = j0 + 32 * kh + n;
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  float* const red_k = (float*)(kh == 0 ? sQ : sK);
+  float* const red_v = (float*)(kh == 0 ? sO : sV);
   if (qc == 1) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        red[(t * 16 + r) * kWave + lane] = acc_dk[t][r];
-        red[((2 + t) * 16 + r) * kWave + lane] = acc_dv[t][r];
+        red_k[(t * 16 + r) * kWave + lane] = acc_dk[t][r];
+        red_v[(t * 16 + r) * kWave + lane] = acc_dv[t][r];
       }
   }
   __syncthreads();
-  if (nparts > 1) {                        // this part's share, added by bwd_sum_kernel
-    if (qc == 0) {
-      float* const pk = a.part_kv + ((((int64_t)b * p.H + h) * a.slot_cap + it.w + it.y) * 2 * kBwIT +
-                                     32 * kh + n) * D + 64 * dh + 4 * hl;
+  if (qc == 1) return;
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          float wk[4], wvv[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int r = 4 * g + j;
-            wk[j] = acc_dk[t][r] + red[(t * 16 + r) * kWave + lane];
-            wvv[j] = acc_dv[t][r] + red[((2 + t) * 16 + r) * kWave + lane];
-          }
-          *(float4*)(pk + 32 * t + 8 * g) = make_float4(wk[0], wk[1], wk[2], wk[3]);
-          *(float4*)(pk + kBwIT * D + 32 * t + 8 * g) = make_float4(wvv[0], wvv[1], wvv[2], wvv[3]);
-        }
+    for (int r = 0; r < 16; ++r) {
+      acc_dk[t][r] += red_k[(t * 16 + r) * kWave + lane];
+      acc_dv[t][r] += red_v[(t * 16 + r) * kWave + lane];
     }
+  if (nparts > 1) {                        // this part's share, added by bwd_sum_kernel
+    float* const pk = a.part_kv + ((((int64_t)b * p.H + h) * a.slot_cap + it.w + it.y) * 2 * kBwIT +
+                                   32 * kh + n) * D + 4 * hl;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        *(float4*)(pk + 32 * t + 8 * g) = make_float4(acc_dk[t][4 * g], acc_dk[t][4 * g + 1],
+                                                      acc_dk[t][4 * g + 2], acc_dk[t][4 * g + 3]);
+        *(float4*)(pk + kBwIT * D + 32 * t + 8 * g) = make_float4(acc_dv[t][4 * g], acc_dv[t][4 * g + 1],
+                                                                  acc_dv[t][4 * g + 2], acc_dv[t][4 * g + 3]);
+      }
     return;
   }
-  if (qc == 0 && key < len) {
+  if (key < len) {
     bf16* dkp = seq_base(a.dk, p.cu, b, a.dk_sb, a.dk_st) + (int64_t)h * a.dk_sh + (int64_t)key * a.dk_st;
     bf16* dvp = seq_base(a.dv, p.cu, b, a.dv_sb, a.dv_st) + (int64_t)h * a.dv_sh + (int64_t)key * a.dv_st;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         bf16x4 wk, wvv;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const int r = 4 * g + j;
-          wk[j] = (bf16)((acc_dk[t][r] + red[(t * 16 + r) * kWave + lane]) * a.scale);
-          wvv[j] = (bf16)(acc_dv[t][r] + red[((2 + t) * 16 + r) * kWave + lane]);
+          wk[j] = (bf16)(acc_dk[t][4 * g + j] * a.scale);
+          wvv[j] = (bf16)acc_dv[t][4 * g + j];
         }
-        *(bf16x4*)(dkp + 64 * dh + 32 * t + 8 * g + 4 * hl) = wk;
-        *(bf16x4*)(dvp + 64 * dh + 32 * t + 8 * g + 4 * hl) = wvv;
+        *(bf16x4*)(dkp + 32 * t + 8 * g + 4 * hl) = wk;
+        *(bf16x4*)(dvp + 32 * t + 8 * g + 4 * hl) = wvv;
       }
   }
 }
