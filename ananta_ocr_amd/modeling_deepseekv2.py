@@ -31,6 +31,8 @@ import torch
 from . import ops, page_rope, pages
 from .dash_attention import DashAttention, apply_rotary, checkpoint_sparse_config
 
+_DASH_FORWARD_TRITON = DashAttention._forward_triton
+
 _INFER = {"on": False}
 
 
@@ -248,9 +250,19 @@ def _infer_prefill_attend(self, router, hidden_states, q, k, v, idx_pe, pos_ids,
         _decode_caches(past_kv)[self.layer_idx] = dc
         past_kv._dash_idx_k[self.layer_idx] = dc.idx_k
     sc = router.block_scores(idx_q, idx_k, q_pos=pos_ids.to(torch.int32), nblk=nblk, kbar=kb)
-    topi, bias, valid = _infer_route_select(sc, block_cand, p)
-    if router.use_triton and q.is_cuda and attn_mask is None:
-        out = router._forward_triton(q, k, v, topi, bias, valid, S, nblk, pos_ids)
+    # _infer_route_select with the ids left in 32 bits, as the attention takes them
+    topi, bias, valid = ops.route(sc, block_cand, p["idx_scale"], p["floor"], p["sigma"], p["K"],
+                                  p["topm"])
+    # Without a mask the kernel entry point and the fallback are the same attention here: the
+    # entry point's test that positions count from 0, which only chooses between them, is a
+    # host synchronisation in the middle of the prefill (with the launches that prepare it
+    # 40 us of GPU work; 296 -> 222 us a layer of 2,730 tokens).  Routers with their own
+    # _forward_triton, and types that the entry point refuses, still go through it.
+    own = getattr(type(router), "_forward_triton", None) is not _DASH_FORWARD_TRITON \
+        or "_forward_triton" in vars(router)
+    if router.use_triton and q.is_cuda and attn_mask is None \
+            and (own or q.dtype != torch.bfloat16):
+        out = router._forward_triton(q, k, v, topi.long(), bias, valid, S, nblk, pos_ids)
         if out is not None:
             return out
     return router._forward_dense(q, k, v, topi, bias, valid, S, nblk, attn_mask)

@@ -136,7 +136,7 @@ def block_cand(pos_ids, num_key_blocks, block_size, image_token_mask=None,
         qpi = query_token_page_ids.to(torch.int32).contiguous()
     elif image_token_mask is not None:
         mode = 1
-        ipi = torch.where(image_token_mask.bool(), 0, -1).to(torch.int32).contiguous()
+        ipi = image_token_mask.bool().to(torch.int32).contiguous().sub(1)   # 0: image, -1: not
         qpi = None
     else:
         mode = 2
