@@ -691,10 +691,19 @@ __device__ __forceinline__ void route_row_topm(const uint32_t (&hi)[NPL], const 
     const uint64_t mt = __ballot(take);
     if (take) sel[lane_prefix(mt)] = mine;
   } else {
-    const uint32_t T = kth_key<NPL>(hi, M, t0, kmax);
+    // Fewer than M entries above t0 make it the M-th largest: rows with few remote or
+    // candidate blocks, whose other entries tie at the floor (a paged prompt of 8,301
+    // tokens: 35 us without this test, 20 with it).
     int n_gt = 0;
 #pragma unroll
-    for (int i = 0; i < NPL; ++i) n_gt += __popcll(__ballot(hi[i] > T));
+    for (int i = 0; i < NPL; ++i) n_gt += __popcll(__ballot(hi[i] > t0));
+    uint32_t T = t0;
+    if (n_gt >= M) {
+      T = kth_key<NPL>(hi, M, t0, kmax);
+      n_gt = 0;
+#pragma unroll
+      for (int i = 0; i < NPL; ++i) n_gt += __popcll(__ballot(hi[i] > T));
+    }
     const int need_eq = M - n_gt;
     int taken = 0, eq_seen = 0;
 #pragma unroll
