@@ -874,86 +874,72 @@ __global__ __launch_bounds__(256, 2) void bwd_q_kernel(BwdArgs a) {
     item(it, std::integral_constant<int, 0>{});
     if (it + 1 < nit) item(it + 1, std::integral_constant<int, 1>{});
   }
-  if (!qvalid) return;
-  // The routed partials of this query (every kept routed slot is block-major), in
-  // slot order and, within a slot, sub-block order.  Slots in groups of 16: the
-  // group's kinds and pair positions are loaded before any is used, then the
-  // partial rows two at a time (both rows' loads in flight before either is added).
-  for (int g0 = 0; p.kind && g0 < p.K; g0 += kPfMaxK) {
-    const int ng = min(kPfMaxK, p.K - g0);
-    const int64_t q0 = qrow * p.K + g0;
-    int32_t pos[kPfMaxK];
-    uint32_t live = 0;
-    if (p.slots_vec) {                     // ng is a multiple of 4
-      uint32_t kw[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const bool in = 4 * q < ng;
-        kw[q] = in ? *(const uint32_t*)(p.kind + q0 + 4 * q) : 0u;
-        const int4 pv = in ? *(const int4*)(p.spos + q0 + 4 * q) : make_int4(-1, -1, -1, -1);
-        pos[4 * q] = pv.x; pos[4 * q + 1] = pv.y; pos[4 * q + 2] = pv.z; pos[4 * q + 3] = pv.w;
-      }
-#pragma unroll
-      for (int s = 0; s < kPfMaxK; ++s)
-        if (((kw[s >> 2] >> (8 * (s & 3))) & 0xffu) == 2 && pos[s] >= 0) live |= 1u << s;
-    } else {
-      uint8_t kd[kPfMaxK];
-#pragma unroll
-      for (int s = 0; s < kPfMaxK; ++s) {
-        kd[s] = s < ng ? p.kind[q0 + s] : 0;
-        pos[s] = s < ng ? p.spos[q0 + s] : -1;
-      }
-#pragma unroll
-      for (int s = 0; s < kPfMaxK; ++s)
-        if (kd[s] == 2 && pos[s] >= 0) live |= 1u << s;
-    }
-    if (!__any(live != 0u)) continue;
-    const int ne = ng * a.nsub;            // (slot, sub-block) rows of the group
-    for (int e0 = 0; e0 < ne; e0 += 2) {
-      f16x4 buf[2][16];
-      float4 sc[2];                        // the scales of the row's four 32-dim pieces
-      bool in[2];
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int e = e0 + q, s = e / a.nsub, u = e - s * a.nsub;
-        in[q] = e < ne && ((live >> s) & 1u);
-        if (in[q]) {
-          const int64_t pr = ((int64_t)h * p.ppos + pos[s]) * a.nsub + u;
-          const _Float16* pd = a.part_dq + pr * D + 64 * hl;
-#pragma unroll
-          for (int k = 0; k < 8; ++k) {
-            const f16x8 w = *(const f16x8*)(pd + 8 * k);
-            buf[q][2 * k] = f16x4{w[0], w[1], w[2], w[3]};
-            buf[q][2 * k + 1] = f16x4{w[4], w[5], w[6], w[7]};
-          }
-          sc[q] = *(const float4*)(a.part_dqs + pr * 4);
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-        if (in[q]) {
-          const float sca[4] = {sc[q].x, sc[q].y, sc[q].z, sc[q].w};
-#pragma unroll
-          for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              const f16x4 v4 = buf[q][4 * dt + g];
-#pragma unroll
-              for (int j = 0; j < 4; ++j) acc_q[dt][4 * g + j] = fmaf((float)v4[j], sca[dt], acc_q[dt][4 * g + j]);
-            }
-        }
-    }
-  }
-  bf16* dqp = seq_base(a.dq, p.cu, b, a.dq_sb, a.dq_st) + (int64_t)h * a.dq_sh + (int64_t)tq * a.dq_st;
+  // The window's dQ passes through LDS (16 KB of the stages per wavefront: 32 rows of 128
+  // fp32 in the partials' dim order, 16-byte chunk c of row r at slot c ^ r), so that 16
+  // lanes hold a query's row and read its partials in whole 256-byte rows.  Read in the
+  // accumulators' layout, a lane took 128 bytes of its own query's partials in eight loads,
+  // whose lines the CU's vector cache did not hold that long: 490 us against 476 for
+  // 27,300 tokens of 16 slots and window 1,024, 206 against 192 for 2 x 2,730 of 64.
+  __syncthreads();                         // every wavefront is done with the stages
+  float* const sa = (float*)(wv == 0 ? sK0 : wv == 1 ? sV0 : wv == 2 ? sK1 : sV1);
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      bf16x4 w;
+    for (int g = 0; g < 4; ++g)
+      *(float4*)(sa + n * D + (((16 * hl + 4 * dt + g) ^ n) << 2)) =
+          make_float4(acc_q[dt][4 * g], acc_q[dt][4 * g + 1], acc_q[dt][4 * g + 2], acc_q[dt][4 * g + 3]);
+  wave_lds_sync();
+  // lane m of 16: places 8 m .. 8 m + 7 of the row, dims d0 .. d0 + 3 and d0 + 8 .. d0 + 11
+  const int m = lane & 15;
+  const int piece = (m & 7) >> 1, d0 = 32 * piece + 16 * (m & 1) + 4 * (m >> 3);
+  for (int pass = 0; pass < 8; ++pass) {
+    const int r = 4 * pass + (lane >> 4), t = t0 + wv * 32 + r;
+    if (!__any(t < len)) break;
+    const int64_t row = r0 + min(t, len - 1);
+    const float4 w0 = *(const float4*)(sa + r * D + (((2 * m) ^ r) << 2));
+    const float4 w1 = *(const float4*)(sa + r * D + (((2 * m + 1) ^ r) << 2));
+    float acc[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+    // the routed partials (every kept slot is block-major), in slot order and, within a
+    // slot, sub-block order; sixteen rows in flight
+    for (int g0 = 0; p.kind && g0 < p.K; g0 += 16) {
+      int pos = -1;
+      if (g0 + m < p.K && t < len && p.kind[row * p.K + g0 + m] == 2) pos = p.spos[row * p.K + g0 + m];
+      if (!__any(pos >= 0)) continue;
+      const int ne = min(16, p.K - g0) * a.nsub;
+      for (int e0 = 0; e0 < ne; e0 += 16) {
+        f16x8 x[16];
+        float sc[16];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = (bf16)(acc_q[dt][4 * g + j] * a.scale);
-      *(bf16x4*)(dqp + 32 * dt + 8 * g + 4 * hl) = w;
+        for (int i = 0; i < 16; ++i) {
+          const int e = e0 + i, s = a.nsub == 1 ? e : e / a.nsub, u = e - s * a.nsub;
+          const int ps = __shfl(pos, (lane & 48) + (s & 15), kWave);
+          sc[i] = 0.f;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) x[i][j] = (_Float16)0.f;
+          if (e < ne && ps >= 0) {
+            const int64_t pr = ((int64_t)h * p.ppos + ps) * a.nsub + u;
+            x[i] = *(const f16x8*)(a.part_dq + pr * D + 8 * m);
+            sc[i] = a.part_dqs[pr * 4 + piece];
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) acc[j] = fmaf((float)x[i][j], sc[i], acc[j]);
+      }
     }
+    if (t < len) {
+      bf16* dqp = seq_base(a.dq, p.cu, b, a.dq_sb, a.dq_st) + (int64_t)h * a.dq_sh + (int64_t)t * a.dq_st + d0;
+      bf16x4 o0, o1;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        o0[j] = (bf16)(acc[j] * a.scale);
+        o1[j] = (bf16)(acc[4 + j] * a.scale);
+      }
+      *(bf16x4*)dqp = o0;
+      *(bf16x4*)(dqp + 8) = o1;
+    }
+  }
 }
 
 // d_bias[row, slot] = sum over heads of the slot's pair partial (0 for slots that
