@@ -67,6 +67,7 @@ SIGNATURES = {
     "dash_attn_decode": (_i, [_p, _l, _l, _p, _l, _l, _l, _l, _p, _l, _l, _l, _l, _p, _l, _i,
                               _p, _p, _p, _p, _p, _i, _p, _i, _l, _l, _p, _l, _l, _i, _i, _i,
                               _i, _i, _i, _f, _i, _p, _l, _p]),
+    "dash_packed_row_blocks": (_i, [_p, _i, _i, _i, _p, _p]),
     "dash_extend_scores": (_i, [_p, _l, _p, _l, _l, _p, _p, _p, _p, _p, _l, _p, _i, _i, _i, _i, _i,
                                 _i, _i, _i, _p, _p, _p, _l, _p]),
     "dash_attn_extend_workspace_size": (_i, [_i, _i, _i, _l, _i, _i, ctypes.POINTER(_l)]),

@@ -1325,7 +1325,8 @@ extern "C" int dash_block_scores(const float* idx_q, int64_t iq_sb, int64_t iq_s
 // ---------------------------------------------------------------------------
 namespace dash {
 // Position and block count of every query row: row cu[b] + i is position ctx[b] + i of
-// sequence b.
+// sequence b.  Without ctx the rows are whole packed documents, whose block counts alone
+// are written.
 __global__ __launch_bounds__(256) void extend_rows_kernel(const int32_t* __restrict__ cu,
                                                           const int32_t* __restrict__ ctx,
                                                           const int32_t* __restrict__ lens, int B,
@@ -1338,10 +1339,21 @@ __global__ __launch_bounds__(256) void extend_rows_kernel(const int32_t* __restr
     const int mid = (b + hi) >> 1;
     if (cu[mid] <= r) b = mid; else hi = mid;
   }
-  q_pos[r] = ctx[b] + r - cu[b];
-  row_nblk[r] = (lens[b] + bs - 1) / bs;
+  if (ctx) q_pos[r] = ctx[b] + r - cu[b];
+  row_nblk[r] = ((ctx ? lens[b] : cu[b + 1] - cu[b]) + bs - 1) / bs;
 }
 }  // namespace dash
+
+extern "C" int dash_packed_row_blocks(const int32_t* cu_seqlens, int B, int T, int block_size,
+                                      int32_t* row_nblk, void* stream) {
+  using namespace dash;
+  if (!cu_seqlens || !row_nblk || B < 0 || T < 0 || block_size <= 0) return kErrInvalid;
+  if (B == 0 || T == 0) return kOk;
+  hipLaunchKernelGGL(extend_rows_kernel, dim3((T + 255) / 256), dim3(256), 0, (hipStream_t)stream,
+                     cu_seqlens, (const int32_t*)nullptr, (const int32_t*)nullptr, B, T, block_size,
+                     (int32_t*)nullptr, row_nblk);
+  return launch_status();
+}
 
 extern "C" int dash_extend_scores(const float* idx_q, int64_t iq_st, const float* idx_k,
                                   int64_t ik_st, int64_t ik_sp, const float* head_cls,

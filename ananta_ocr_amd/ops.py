@@ -907,6 +907,18 @@ def attn_rows(q, k, v, idx, bias, valid, q_pos, row_seq, block_size, local_windo
     return out
 
 
+def packed_row_blocks(cu_seqlens, rows, block_size):
+    """Block count [rows] int32 of every token row's document (packed documents of
+    cu_seqlens[-1] = rows tokens on the GPU), in one launch without a host read."""
+    _need_gpu(cu_seqlens)
+    cu = _i32(cu_seqlens)
+    out = torch.empty(rows, dtype=torch.int32, device=cu.device)
+    _lib.check(_lib.load().dash_packed_row_blocks(_ptr(cu), cu.numel() - 1, int(rows),
+                                                  int(block_size), _ptr(out), _stream()),
+               "dash_packed_row_blocks")
+    return out
+
+
 def extend_scores_ok(idx_q, idx_k, pool, block_size):
     """Whether extend_scores takes these index queries, paged index keys and k_bar pool."""
     return (idx_q.dim() == 2 and idx_k.dim() == 3 and idx_q.shape[-1] == idx_k.shape[-1] == 128

@@ -27,9 +27,7 @@ def prefill(q, k, v, idx_q, idx_k, head_cls, block_size, local_blocks, idx_scale
     z = ops.block_scores(idx_q, kb, block_size, local_blocks, cu_seqlens=cu_seqlens,
                          max_seqlen=max_seqlen)
     if cu_seqlens is not None:
-        lens = (cu_seqlens[1:] - cu_seqlens[:-1]).to(torch.int32)
-        nblk_doc = (lens + block_size - 1) // block_size
-        row_nblk = torch.repeat_interleave(nblk_doc, lens.long(), output_size=z.shape[0])
+        row_nblk = ops.packed_row_blocks(cu_seqlens, z.shape[0], block_size)
         width = max(1, min(int(K), int(topm))) if int(topm) > 0 else max(1, int(K))
         idx, bias, valid = ops.route(z, block_cand, idx_scale, floor, sigma, K, topm,
                                      row_nblk=row_nblk, width=width)

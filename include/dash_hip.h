@@ -411,6 +411,11 @@ int dash_extend_scores(const float* idx_q, int64_t iq_st, const float* idx_k, in
                        int block_size, int local_blocks, int32_t* q_pos, int32_t* row_nblk,
                        float* z, int64_t z_stride, void* stream);
 
+/* Blocks of the document of every token row of packed documents cu_seqlens [B + 1] with
+ * T = cu_seqlens[B] rows: row_nblk [T], as dash_route takes it. */
+int dash_packed_row_blocks(const int32_t* cu_seqlens, int B, int T, int block_size,
+                           int32_t* row_nblk, void* stream);
+
 /* Workspace bytes dash_attn_extend needs. */
 int dash_attn_extend_workspace_size(int B, int H, int max_query_len, int64_t T, int K, int nblk,
                                     int64_t* bytes);

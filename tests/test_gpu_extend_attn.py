@@ -159,3 +159,11 @@ def test_extend_scores_equal_the_general_path():
     ref = ops.block_scores(iq[None], kb, bs, lb, q_pos=q_pos, cu_seqlens=cu, max_seqlen=max(news),
                            key_lens=ln, S=P * bs)
     assert torch.equal(z, ref)
+
+
+@pytest.mark.parametrize("lens", [[1], [64, 1, 65], [300, 0, 0, 31], [0, 200, 257]])
+def test_packed_row_blocks(lens):
+    cu = torch.tensor([0] + lens).cumsum(0).to(DEV)
+    n = torch.tensor(lens)
+    ref = torch.repeat_interleave((n + 63) // 64, n).to(torch.int32)
+    assert torch.equal(ops.packed_row_blocks(cu, sum(lens), 64).cpu(), ref)
