@@ -177,11 +177,10 @@ def block_max_score(q, k, pos, seg, block_size, num_key_blocks, local_window, mo
     return out
 
 
-# Fewest query rows per sequence for the matrix-core block-max kernel, which splits every key
-# into bf16 parts first and works on 128 rows at a time.  2,730 keys in blocks of 32: 128 rows
-# 22.8 us against 19.8 us row by row, 2,730 rows 25.5 against 96.4; 27,300 rows and keys 551
-# against 7,514 us.
-BLOCK_MAX_FUSED_ROWS = 256
+# Fewest query rows per sequence for the matrix-core block-max kernel, which gives the bits of
+# the row-by-row kernel: any number.  389 to 27,300 keys, batches of 1 and 8, blocks of 32 and
+# 64: 1 row 10.5 to 56 us against 16 to 144 row by row, 2,730 rows of 2,730 keys 26 against 94.
+BLOCK_MAX_FUSED_ROWS = 1
 
 
 def _block_max_fused_ok(d, block_size):
@@ -200,15 +199,19 @@ def _block_max_fused(q, k, pos, seg, block_size, nblk, lw, mode, want_arg=False)
     lib = _lib.load()
     q, k = _f4_rows(q), _f4_rows(k)
     B, C, d = q.shape
-    nbytes = ctypes.c_int64(0)
-    _lib.check(lib.dash_block_max_fused_workspace_size(B, block_size, nblk, nbytes), "workspace")
-    ws = torch.empty(max(nbytes.value, 16), dtype=torch.uint8, device=q.device)
+    ws = None
+    if mode == 2:
+        nbytes = ctypes.c_int64(0)
+        _lib.check(lib.dash_block_max_fused_workspace_size(B, block_size, nblk, nbytes),
+                   "workspace")
+        ws = torch.empty(max(nbytes.value, 16), dtype=torch.uint8, device=q.device)
     out = torch.empty(B, C, nblk, dtype=torch.float32, device=q.device)
     arg = torch.empty(B, C, nblk, dtype=torch.uint8, device=q.device) if want_arg else None
     st_ = lib.dash_block_max_fused(
         _ptr(q), q.stride(0), q.stride(1), C, _ptr(pos), _ptr(seg), pos.stride(0), _ptr(k),
         k.stride(0), k.stride(1), k.shape[1], B, d, block_size, lw, nblk, mode, _ptr(out),
-        out.stride(0), out.stride(1), _ptr(arg), _ptr(ws), ws.numel(), _stream())
+        out.stride(0), out.stride(1), _ptr(arg), _ptr(ws), 0 if ws is None else ws.numel(),
+        _stream())
     _lib.check(st_, "dash_block_max_fused")
     return out, arg
 

@@ -89,10 +89,11 @@ int dash_block_max_score(const float* q, int64_t q_sb, int64_t q_st, int C,
 
 /*
  * The same scores on the matrix cores: d = 128, block_size 32, 64, 96 or 128, rows of q and
- * k 16-byte aligned (strides multiples of 4); else unsupported.  mode 2 = the training form
- * (mode 0, but a NaN score makes its block's score NaN).  arg [B, C, nblk] (or NULL): the
- * winning key of every block, within the block, 255 where there is no single one; the
- * backward call reads it.  ws: 16-byte aligned, of the size
+ * k 16-byte aligned (strides multiples of 4); else unsupported.  Modes 0 and 1 give the bits
+ * of dash_block_max_score.  mode 2 = the training form (mode 0, but a NaN score makes its
+ * block's score NaN), with sums in another order.  arg [B, C, nblk] (or NULL): the winning
+ * key of every block, within the block, 255 where there is no single one; the backward call
+ * reads it.  ws (mode 2, or with arg; else NULL): 16-byte aligned, of the size
  * dash_block_max_fused_workspace_size gives; its contents need not be kept.
  */
 int dash_block_max_fused_workspace_size(int B, int block_size, int nblk, int64_t* bytes);

@@ -112,6 +112,36 @@ def test_scores_of_values_that_are_not_finite(mode, monkeypatch):
     assert torch.equal(out[~fin & ~old.isnan()], old[~fin & ~old.isnan()])
 
 
+@pytest.mark.parametrize("values", ["normal", "tiny", "large", "spread", "special"])
+@pytest.mark.parametrize("B,C,Sk,bs,lw,mode", [(1, 1, 389, 32, 128, 0), (2, 129, 500, 96, 1, 1),
+                                               (1, 300, 1111, 64, 100, 1), (1, 900, 900, 32, 1, 0),
+                                               (1, 257, 2500, 128, 128, 0)])
+def test_scores_are_the_row_by_row_bits(B, C, Sk, bs, lw, mode, values, monkeypatch):
+    """A row's inference scores are the same bits in a call of any number of rows: whole
+    prompts, chunks and decode steps route rows that all but tie alike."""
+    g = torch.Generator().manual_seed(C + bs)
+    q, k = torch.randn(B, C, 128, generator=g), torch.randn(B, Sk, 128, generator=g)
+    if values == "tiny":                            # sums below the smallest normal value
+        q, k = q * 1e-20, k * 1e-19
+    elif values == "large":                         # sums that overflow
+        q, k = q * 1e18, k * 1e20
+    elif values == "spread":                        # the order of the sum shows in every bit
+        q = q * (12 * torch.randn(q.shape, generator=g)).exp()
+        k = k * (12 * torch.randn(k.shape, generator=g)).exp()
+    elif values == "special":
+        q[0, 0, 3], k[0, 33, 7], k[0, 95, 0] = math.inf, -math.inf, math.nan
+        k[0, 200:216], k[0, 300], k[0, 301] = 3.0e38, 0.0, 1e-42
+        q[0, C // 2] = 0.0
+    pos = torch.arange(Sk - C, Sk).expand(B, C)
+    seg = (pos // 3).to(DEV) if mode == 1 else None
+    nblk = (Sk + bs - 1) // bs + 1
+    args = (q.to(DEV), k.to(DEV), pos.to(DEV), seg, bs, nblk, lw)
+    out = ops.block_max_score(*args, mode=mode)
+    monkeypatch.setattr(ops, "BLOCK_MAX_FUSED_ROWS", C + 1)
+    old = ops.block_max_score(*args, mode=mode)
+    assert torch.equal(out.view(torch.int32), old.view(torch.int32))
+
+
 def test_gradient_of_the_gradient():
     """create_graph goes through the tensor ops."""
     r = _router(32, 1)
