@@ -157,7 +157,7 @@ def block_scores(idx_q, kb, block_size, local_blocks, q_pos=None, cu_seqlens=Non
 def block_max_score(q, k, pos, seg, block_size, num_key_blocks, local_window, mode=1):
     """Indexer block-max scores (mode 1: triton_block_max_score semantics, mode 0:
     the torch indexer form).  q [B,C,d], k [B,Sk,d] fp32; pos/seg [B,C]."""
-    _need_gpu(q, k, pos)
+    _need_gpu(q, k, pos, seg)
     lib = _lib.load()
     q = q.float().contiguous()
     k = k.float().contiguous()
@@ -196,6 +196,7 @@ def _f4_rows(x):
 
 def _block_max_fused(q, k, pos, seg, block_size, nblk, lw, mode, want_arg=False):
     """dash_block_max_fused: (scores [B,C,nblk] fp32, winning keys uint8 or None)."""
+    _need_gpu(q, k, pos, seg)
     lib = _lib.load()
     q, k = _f4_rows(q), _f4_rows(k)
     B, C, d = q.shape
@@ -267,6 +268,7 @@ def block_max_train(iq, ik, position_ids, block_size, local_window, nblk, differ
     max over each block's keys j <= position - local_window of clamp(iq . ik_j, +-1e4),
     -1e9 where there is none, with autograd to iq and ik.  differentiable(iq, ik,
     position_ids, nblk): the same scores by tensor ops, for a graph of the gradient."""
+    _need_gpu(iq, ik, position_ids)
     pos = _i32(position_ids.expand(iq.shape[:2]))
     return _BlockMaxFn.apply(iq, ik, pos, block_size, int(local_window), nblk, differentiable)
 

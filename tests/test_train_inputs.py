@@ -1,0 +1,39 @@
+"""Inputs of the training front end and indexer scores that the library refuses or takes in
+another way, checked on the CPU before any launch."""
+
+import pytest
+import torch
+
+from ananta_ocr_amd import ops
+
+
+class OnGpu(torch.Tensor):
+    """A CPU tensor that says it is on the GPU: what follows the device checks then fails
+    here instead of reading a host pointer."""
+
+    @property
+    def is_cuda(self):
+        return True
+
+
+def _gpu(*shape):
+    return torch.zeros(*shape).as_subclass(OnGpu)
+
+
+def _no_launch(monkeypatch):
+    def load():
+        raise AssertionError("the library was reached")
+    monkeypatch.setattr(ops._lib, "load", load)
+
+
+def test_positions_in_host_memory_are_refused(monkeypatch):
+    _no_launch(monkeypatch)
+    iq, ik = _gpu(1, 64, 128), _gpu(1, 64, 128)
+    pos = torch.arange(64)[None]
+    assert ops.block_max_train_ok(iq, ik, 32)
+    with pytest.raises(ValueError, match="GPU tensors"):
+        ops.block_max_train(iq, ik, pos, 32, 32, 2, None)
+    with pytest.raises(ValueError, match="GPU tensors"):
+        ops.block_max_train(iq, torch.zeros(1, 64, 128), pos.as_subclass(OnGpu), 32, 32, 2, None)
+    with pytest.raises(ValueError, match="GPU tensors"):
+        ops.block_max_score(iq, ik, pos.as_subclass(OnGpu), pos, 32, 2, 32)
