@@ -266,10 +266,11 @@ class _BlockMaxFn(torch.autograd.Function):
 def block_max_train(iq, ik, position_ids, block_size, local_window, nblk, differentiable):
     """Training indexer scores z [B,S,nblk] fp32 of index queries / keys [B,S,128] fp32:
     max over each block's keys j <= position - local_window of clamp(iq . ik_j, +-1e4),
-    -1e9 where there is none, with autograd to iq and ik.  differentiable(iq, ik,
-    position_ids, nblk): the same scores by tensor ops, for a graph of the gradient."""
+    -1e9 where there is none, with autograd to iq and ik.  position_ids [B or 1, >= S] (the
+    first S columns count).  differentiable(iq, ik, position_ids, nblk): the same scores by
+    tensor ops, for a graph of the gradient."""
     _need_gpu(iq, ik, position_ids)
-    pos = _i32(position_ids.expand(iq.shape[:2]))
+    pos = _i32(position_ids[:, :iq.shape[1]].expand(iq.shape[:2]))
     return _BlockMaxFn.apply(iq, ik, pos, block_size, int(local_window), nblk, differentiable)
 
 

@@ -37,3 +37,16 @@ def test_positions_in_host_memory_are_refused(monkeypatch):
         ops.block_max_train(iq, torch.zeros(1, 64, 128), pos.as_subclass(OnGpu), 32, 32, 2, None)
     with pytest.raises(ValueError, match="GPU tensors"):
         ops.block_max_score(iq, ik, pos.as_subclass(OnGpu), pos, 32, 2, 32)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 64), (2, 64), (1, 100), (2, 65)])
+def test_positions_beyond_the_sequence_are_left_out(rows, cols, monkeypatch):
+    """The tensor ops slice position_ids to the queries, so longer ones are taken."""
+    got = []
+    monkeypatch.setattr(ops._BlockMaxFn, "apply", lambda *a: got.append(a))
+    iq = _gpu(2, 64, 128)
+    pos = torch.arange(rows * cols).view(rows, cols)
+    ops.block_max_train(iq, iq, pos.as_subclass(OnGpu), 32, 32, 2, None)
+    (call,) = got
+    assert torch.equal(call[2].as_subclass(torch.Tensor), pos[:, :64].expand(2, 64).int())
+    assert call[2].is_contiguous()
