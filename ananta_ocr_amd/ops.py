@@ -241,9 +241,11 @@ class _BlockMaxFn(torch.autograd.Function):
         iq, ik, pos, arg = ctx.saved_tensors
         block_size, lw, nblk, differentiable = ctx.cfg
         if torch.is_grad_enabled():            # create_graph: by tensor ops
-            g = torch.autograd.grad(differentiable(iq, ik, pos, nblk), (iq, ik), dz,
-                                    create_graph=True)
-            return (*g, None, None, None, None, None)
+            need = ctx.needs_input_grad[:2]
+            got = iter(torch.autograd.grad(differentiable(iq, ik, pos, nblk),
+                                           [t for t, n in zip((iq, ik), need) if n], dz,
+                                           create_graph=True))
+            return (*[next(got) if n else None for n in need], None, None, None, None, None)
         lib = _lib.load()
         q, k, dz = _f4_rows(iq), _f4_rows(ik), dz.float()
         if dz.stride(-1) != 1:

@@ -50,3 +50,20 @@ def test_positions_beyond_the_sequence_are_left_out(rows, cols, monkeypatch):
     (call,) = got
     assert torch.equal(call[2].as_subclass(torch.Tensor), pos[:, :64].expand(2, 64).int())
     assert call[2].is_contiguous()
+
+
+@pytest.mark.parametrize("leaf", [0, 1])
+def test_gradient_of_the_gradient_of_one_operand(leaf, monkeypatch):
+    """create_graph where only the queries or only the keys require a gradient, as with one
+    projection frozen."""
+    monkeypatch.setattr(ops, "_block_max_fused", lambda q, k, *a, **kw: (q @ k.mT, None))
+    x = [torch.randn(1, 8, 128) for _ in range(2)]
+    x[leaf].requires_grad_()
+    z = ops._BlockMaxFn.apply(*x, None, 32, 32, 8, lambda iq, ik, pos, nblk: (iq @ ik.mT).square())
+    (g,) = torch.autograd.grad(z, x[leaf], torch.ones_like(z), create_graph=True)
+    (gg,) = torch.autograd.grad(g.square().sum(), x[leaf])
+    y = [t.detach().clone() for t in x]
+    y[leaf].requires_grad_()
+    (h,) = torch.autograd.grad((y[0] @ y[1].mT).square().sum(), y[leaf], create_graph=True)
+    (hh,) = torch.autograd.grad(h.square().sum(), y[leaf])
+    assert torch.equal(g, h) and torch.equal(gg, hh)
