@@ -433,8 +433,10 @@ class _RouterFrontFn(torch.autograd.Function):
         need = ctx.needs_input_grad
         if torch.is_grad_enabled():            # create_graph: by tensor ops
             leaves = [t for t, n in zip((hs, w_q, w_k, nq, nk), need) if n]
-            got = iter(torch.autograd.grad(differentiable(hs, w_q, w_k, nq, nk, cos, sin, eps),
-                                           leaves, (d_iq, d_ik), create_graph=True))
+            outs = differentiable(hs, w_q, w_k, nq, nk, cos, sin, eps)
+            # with one side frozen, only the other's output has a graph
+            outs, grads = zip(*[(o, g) for o, g in zip(outs, (d_iq, d_ik)) if o.requires_grad])
+            got = iter(torch.autograd.grad(outs, leaves, grads, create_graph=True))
             return (*[next(got) if n else None for n in need[:5]], None, None, None, None)
         lib = _lib.load()
         B, S, hid = hs.shape

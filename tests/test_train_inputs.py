@@ -1,9 +1,12 @@
 """Inputs of the training front end and indexer scores that the library refuses or takes in
 another way, checked on the CPU before any launch."""
 
+from types import SimpleNamespace
+
 import pytest
 import torch
 
+from ananta_ocr_amd import dash_attention as DA
 from ananta_ocr_amd import ops
 
 
@@ -67,3 +70,27 @@ def test_gradient_of_the_gradient_of_one_operand(leaf, monkeypatch):
     (h,) = torch.autograd.grad((y[0] @ y[1].mT).square().sum(), y[leaf], create_graph=True)
     (hh,) = torch.autograd.grad(h.square().sum(), y[leaf])
     assert torch.equal(g, h) and torch.equal(gg, hh)
+
+
+@pytest.mark.parametrize("need", [(0, 1, 0, 1, 0), (0, 0, 1, 0, 0), (1, 0, 0, 0, 0)])
+def test_front_gradient_of_the_gradient_with_one_side_frozen(need):
+    """create_graph where only the query or only the key side (or only the hidden states)
+    requires a gradient."""
+    g = torch.Generator().manual_seed(1)
+    x = [torch.randn(1, 8, 128, generator=g), *(torch.randn(128, 128, generator=g) / 11 for _ in "qk"),
+         *(torch.randn(128, generator=g) * 0.1 for _ in "qk")]
+    for t, n in zip(x, need):
+        t.requires_grad_(bool(n))
+    grads = [torch.randn(1, 8, 128, generator=g) for _ in range(2)]
+    ctx = SimpleNamespace(saved_tensors=(*x, None, None, None), cfg=(1e-6, DA._front_train_ops),
+                          needs_input_grad=tuple(map(bool, need)) + (False,) * 4)
+    got = ops._RouterFrontFn.backward(ctx, *grads)
+    leaves = [t for t, n in zip(x, need) if n]
+    out = DA._front_train_ops(*x, None, None, 1e-6)
+    loss = sum((o * d).sum() for o, d in zip(out, grads))
+    ref = torch.autograd.grad(loss, leaves, create_graph=True)
+    assert [t is not None for t in got[:5]] == [bool(n) for n in need]
+    for a, b in zip([t for t in got if t is not None], ref):
+        torch.testing.assert_close(a, b)
+        (c,) = torch.autograd.grad(a.square().sum(), leaves[0], retain_graph=True)
+        assert c.isfinite().all() and c.abs().max() > 0
