@@ -187,10 +187,17 @@ def _block_max_fused_ok(d, block_size):
     return d == 128 and block_size in (32, 64, 96, 128)
 
 
+def _aligned(x):
+    """x contiguous from a 16-byte boundary on: a copy where it is a view at another place
+    of a larger buffer, which contiguous() returns as it is."""
+    x = x.contiguous()
+    return x if x.data_ptr() % 16 == 0 else x.clone()
+
+
 def _f4_rows(x):
     """fp32 rows the float4 loads take: contiguous features, 16-byte aligned rows."""
     if x.stride(-1) != 1 or any(s % 4 for s in x.stride()[:-1]) or x.data_ptr() % 16:
-        x = x.contiguous()
+        x = _aligned(x)
     return x
 
 

@@ -142,6 +142,24 @@ def test_scores_are_the_row_by_row_bits(B, C, Sk, bs, lw, mode, values, monkeypa
     assert torch.equal(out.view(torch.int32), old.view(torch.int32))
 
 
+def test_rows_off_a_16_byte_boundary():
+    """Index queries and keys that are views at an odd place of a flat buffer."""
+    g = torch.Generator().manual_seed(9)
+    flat = torch.randn(2 * 300 * 128 + 1, generator=g).to(DEV)
+    q, k = (flat[1 + i * 300 * 128:][:300 * 128].view(1, 300, 128) for i in range(2))
+    pos = torch.arange(300, device=DEV)[None]
+    args = (pos, None, 32, 10, 32)
+    assert torch.equal(ops.block_max_score(q, k, *args, mode=0),
+                       ops.block_max_score(q.clone(), k.clone(), *args, mode=0))
+    out = []
+    for x in ((q, k), (q.clone(), k.clone())):
+        a, b = (t.detach().requires_grad_() for t in x)
+        z = ops.block_max_train(a, b, pos, 32, 32, 10, None)
+        out.append((z, *torch.autograd.grad(z.square().sum() * 1e-9, (a, b))))
+    for x, y in zip(*out):
+        assert torch.equal(x, y)
+
+
 def test_gradient_of_the_gradient():
     """create_graph goes through the tensor ops."""
     r = _router(32, 1)

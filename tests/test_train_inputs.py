@@ -94,3 +94,14 @@ def test_front_gradient_of_the_gradient_with_one_side_frozen(need):
         torch.testing.assert_close(a, b)
         (c,) = torch.autograd.grad(a.square().sum(), leaves[0], retain_graph=True)
         assert c.isfinite().all() and c.abs().max() > 0
+
+
+@pytest.mark.parametrize("offset", [0, 1, 2, 4])
+def test_float_rows_at_any_offset_of_a_buffer(offset):
+    """Rows for 16-byte loads: a contiguous view that starts off a 16-byte boundary is copied."""
+    flat = torch.arange(2 * 5 * 128 + 8.0)
+    assert flat.data_ptr() % 16 == 0
+    x = flat[offset:offset + 1280].view(2, 5, 128)
+    y = ops._f4_rows(x)
+    assert torch.equal(x, y) and y.data_ptr() % 16 == 0 and y.is_contiguous()
+    assert (y.data_ptr() == x.data_ptr()) == (offset % 4 == 0)
