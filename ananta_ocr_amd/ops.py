@@ -411,6 +411,12 @@ def router_front_train_ok(hs, w_q, w_k, nq, nk, cos, sin):
             and not (cos.requires_grad or sin.requires_grad))
 
 
+def _front_rows(hs):
+    """_rows, with a copy of contiguous rows that start off a 16-byte boundary."""
+    x = _rows(hs)
+    return x if x.data_ptr() % 16 == 0 else _aligned(x)
+
+
 class _RouterFrontFn(torch.autograd.Function):
     """Training router front end (dash_attention.py:808-821): idx_q, idx_k [B,S,128] fp32 of
     bf16 hidden states, with the gradient sanitizer on both."""
@@ -419,8 +425,9 @@ class _RouterFrontFn(torch.autograd.Function):
     def forward(ctx, hs, w_q, w_k, nq, nk, cos, sin, eps, differentiable):
         lib = _lib.load()
         B, S, hid = hs.shape
-        x, wq, wk = _rows(hs), w_q.contiguous(), w_k.contiguous()
-        nqf, nkf = nq.float().contiguous(), nk.float().contiguous()
+        x = _front_rows(hs)
+        # parameters may be views at any place of a flat buffer
+        wq, wk, nqf, nkf = (_aligned(t) for t in (w_q, w_k, nq.float(), nk.float()))
         cs, args = _front_cos_sin(cos, sin)
         iq, ik = (torch.empty(B, S, 128, dtype=torch.float32, device=hs.device) for _ in range(2))
         proj = torch.empty(B * S, 256, dtype=torch.bfloat16, device=hs.device)
@@ -448,11 +455,10 @@ class _RouterFrontFn(torch.autograd.Function):
         lib = _lib.load()
         B, S, hid = hs.shape
         dev = hs.device
-        x = _rows(hs.reshape(B * S, hid))
-        wq, wk = w_q.contiguous(), w_k.contiguous()
-        nqf, nkf = nq.float().contiguous(), nk.float().contiguous()
+        x = _front_rows(hs.reshape(B * S, hid))
+        wq, wk, nqf, nkf = (_aligned(t) for t in (w_q, w_k, nq.float(), nk.float()))
         cs, args = _front_cos_sin(cos, sin)
-        gq, gk = (g.float().contiguous() for g in (d_iq, d_ik))
+        gq, gk = (_aligned(g.float()) for g in (d_iq, d_ik))
         dwq = torch.empty_like(wq) if need[1] else None
         dwk = torch.empty_like(wk) if need[2] else None
         dn = torch.empty(2, 128, dtype=torch.float32, device=dev)

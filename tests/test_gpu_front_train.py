@@ -97,6 +97,27 @@ def test_front_train_guards_and_layouts():
     assert torch.autograd.grad(first.float().sum(), x[1])[0].isfinite().all()
 
 
+@pytest.mark.parametrize("which", range(5))
+def test_front_train_parameters_in_a_flat_buffer(which):
+    """Hidden states, a projection or a norm weight at an odd place of a flat buffer, in bf16
+    and (norm weights) fp32: the same bits as from its own buffer, forward and backward."""
+    leaves, cos, sin, gr = _inputs(2, 70, 256, torch.bfloat16, 2)
+    for dtype in [torch.bfloat16] + [torch.float32] * (which > 2):
+        x = [t.to(dtype) if i == which else t for i, t in enumerate(leaves)]
+        got = []
+        for odd in (False, True):
+            y = [t.detach().clone() for t in x]
+            if odd:
+                flat = torch.zeros(x[which].numel() + 1, dtype=dtype, device=DEV)
+                y[which] = flat[1:].view(x[which].shape).copy_(x[which])
+            y = [t.requires_grad_() for t in y]
+            assert ops.router_front_train_ok(*y, cos, sin)
+            out = ops.router_front_train(*y, 1e-6, cos, sin, DA._front_train_ops)
+            got.append(list(out) + list(torch.autograd.grad(out, y, gr)))
+        for a, b in zip(*got):
+            assert torch.equal(a, b)
+
+
 def test_front_train_leaves_wrapped_modules_alone():
     """A projection with a hook, or replaced, runs as a module."""
     r = DA.DashAttention(__import__("types").SimpleNamespace(
