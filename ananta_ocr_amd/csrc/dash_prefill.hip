@@ -1754,7 +1754,7 @@ namespace dash {
 struct BwdLayout {
   PlanLayout P;
   int64_t pdb, pdq, pdqs, delta, items, nitems, sparts, pkv, total;
-  int nstage, part_steps, item_cap, slot_cap;
+  int nstage, part_steps, item_cap, per;
 };
 // Steps of a part of a key-major stage, at least; a stage's window steps count double where
 // they are more, so that the stages in parts are those of many pairs.  A fifth of a CU's even
@@ -1776,18 +1776,17 @@ inline BwdLayout bwd_layout(int B, int H, int S_max, int64_t rows, int K, int D,
   L.nstage = (int)(((int64_t)nblk_cap * bs + kBwIT - 1) / kBwIT);
   // stages that take a block's pairs
   const int64_t per = bs <= kBwIT ? 1 : bs % kBwIT == 0 ? nsub : nsub + 1;
+  L.per = (int)per;
   const int64_t est = H * (per * rows * K / kBwIT + rows / kBwIT + B) / (256 * 5);
   L.part_steps = (int)std::min<int64_t>(std::max<int64_t>(est, kBwMinSteps), kBwMaxSteps);
-  // a stage in parts of X steps has more than X / 2 steps of pairs (r), so at most
-  // (r + X / 2) / X + 1 <= 4 r / X parts
+  // parts - 1 < 2 r / X for a stage with r steps of pairs (see part_slots)
   const int64_t pair_steps = K > 0 ? per * ((int64_t)S_max * K / kBwIT + nblk_cap) : 0;
-  const int64_t slots = 4 * pair_steps / L.part_steps + 1;
-  L.slot_cap = (int)slots;
-  L.item_cap = (int)(L.nstage + 2 * pair_steps / L.part_steps + 1);   // parts - 1 < 2 r / X
+  L.item_cap = (int)(L.nstage + 2 * pair_steps / L.part_steps + 1);
+  const int64_t slots = K > 0 ? part_slots(rows, B, K, bs, per, L.part_steps) + 1 : 0;
   L.items = o; o = align256(o + (int64_t)B * L.item_cap * 16);
   L.nitems = o; o = align256(o + (int64_t)B * 4);
   L.sparts = o; o = align256(o + (int64_t)B * L.nstage * 8);
-  L.pkv = o; o = align256(o + (int64_t)B * H * L.slot_cap * 2 * kBwIT * D * 4);
+  L.pkv = o; o = align256(o + slots * H * 2 * kBwIT * D * 4);
   L.total = o;
   return L;
 }
@@ -2034,7 +2033,7 @@ extern "C" int dash_attn_prefill_backward(
   a.nsub = (block_size + kBwIT - 1) / kBwIT;
   a.nstage = L.nstage;
   a.part_steps = std::max(L.part_steps, 2 * ((kBwIT - 2 + local_window) / kBwIT + 1));
-  a.item_cap = L.item_cap; a.slot_cap = L.slot_cap;
+  a.item_cap = L.item_cap; a.per = L.per;
   a.items = (int4*)(w + L.items);
   a.n_items = (int32_t*)(w + L.nitems);
   a.stage_parts = (int2*)(w + L.sparts);

@@ -55,11 +55,12 @@ struct BwdArgs {
   // key-major work list (bwd_items_kernel): a stage of more than part_steps steps is cut
   // into parts, whose dK and dV go to part_kv in fp32 and are added by bwd_sum_kernel
   int part_steps;
-  int item_cap, slot_cap;                 // items and part slots per sequence
+  int item_cap;                           // items per sequence
+  int per;                                // stages that take a block's pairs
   int4* items;                            // [B, item_cap] stage, part, parts, first slot
   int32_t* n_items;                       // [B]
   int2* stage_parts;                      // [B, nstage] first slot, parts (0: nothing to add)
-  float* part_kv;                         // [B, H, slot_cap, 2, 64, 128] dK (not scaled), dV
+  float* part_kv;                         // [slots, H, 2, 64, 128] dK (not scaled), dV
   int nsub;                               // 64-key stages per block (1 for blocks <= 64 keys)
 };
 
@@ -293,6 +294,17 @@ __device__ __forceinline__ KvSteps kv_steps(const PrefillArgs& p, int b, int len
   return k;
 }
 
+// The sequences' part slots lie one after the other in one pool, sequence b's from
+// part_slots(rows before it, b) on.  A stage in parts of X steps has more than X / 2 steps of
+// pairs (r), so at most (r + X / 2) / X + 1 <= 4 r / X parts; a sequence of n rows has at most
+// P (n K / 64 + n / bs + 1) such steps (P stages take a block's pairs), and the floors of
+// prefix sums leave each sequence the floor of its own share.  (A pool per sequence, sized for
+// the longest, took 40 GB for 256 documents of which one has 27,300 tokens.)
+__host__ __device__ inline int64_t part_slots(int64_t rows, int64_t seqs, int K, int bs, int64_t per,
+                                              int64_t part_steps) {
+  return 4 * per * (rows * K * bs + 64 * rows + 64 * seqs * bs) / (64 * bs * part_steps);
+}
+
 // Work list of the key-major kernel, one work-group per sequence: its stages in order, each
 // in ceil(steps / part_steps) parts.  A block that most queries route to (the first blocks,
 // where zero priors tie) has hundreds of steps, which one work-group took alone while the
@@ -302,7 +314,7 @@ __global__ __launch_bounds__(256) void bwd_items_kernel(BwdArgs a) {
   const PrefillArgs& p = a.p;
   const int b = blockIdx.x, tid = threadIdx.x, lane = wave_lane(), wv = tid / kWave;
   const int len = seq_len(p, b);
-  int item0 = 0, slot0 = 0;
+  int item0 = 0, slot0 = (int)part_slots(row0(p, b), b, p.K, p.bs, a.per, a.part_steps);
   for (int s0 = 0; s0 < a.nstage; s0 += 256) {
     const int stage = s0 + tid, j0 = stage * kBwIT;
     int parts = 0;
@@ -327,7 +339,7 @@ __global__ __launch_bounds__(256) void bwd_items_kernel(BwdArgs a) {
     __syncthreads();
     const int fi = item0 + xi - parts, fs = slot0 + xs - slots;
     for (int q = 0; q < parts; ++q)
-      if (fi + q < a.item_cap)             // always, as are the slots below slot_cap
+      if (fi + q < a.item_cap)             // always
         a.items[(int64_t)b * a.item_cap + fi + q] = make_int4(stage, q, parts, fs);
     if (stage < a.nstage) a.stage_parts[(int64_t)b * a.nstage + stage] = make_int2(fs, slots);
     item0 += ti;
@@ -703,8 +715,7 @@ __global__ __launch_bounds__(256, 2) void bwd_kv_kernel(BwdArgs a) {
       acc_dv[t][r] += red_v[(t * 16 + r) * kWave + lane];
     }
   if (nparts > 1) {                        // this part's share, added by bwd_sum_kernel
-    float* const pk = a.part_kv + ((((int64_t)b * p.H + h) * a.slot_cap + it.w + it.y) * 2 * kBwIT +
-                                   32 * kh + n) * D + 4 * hl;
+    float* const pk = a.part_kv + (((int64_t)(it.w + it.y) * p.H + h) * 2 * kBwIT + 32 * kh + n) * D + 4 * hl;
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -744,13 +755,13 @@ __global__ __launch_bounds__(256) void bwd_sum_kernel(BwdArgs a) {
   const int2 sp = a.stage_parts[(int64_t)b * a.nstage + stage];
   if (sp.y == 0) return;
   const int len = seq_len(p, b);
-  const float4* src = (const float4*)(a.part_kv + (((int64_t)b * p.H + h) * a.slot_cap + sp.x) * 2 * kBwIT * D);
+  const float4* src = (const float4*)(a.part_kv + ((int64_t)sp.x * p.H + h) * 2 * kBwIT * D);
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int e = (blockIdx.x & 3) * 1024 + u * 256 + threadIdx.x;   // float4 of the 2 x 64 x 32
     float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int q = 0; q < sp.y; ++q) {
-      const float4 x = src[(int64_t)q * 2 * kBwIT * (D / 4) + e];
+      const float4 x = src[(int64_t)q * p.H * 2 * kBwIT * (D / 4) + e];
       s.x += x.x; s.y += x.y; s.z += x.z; s.w += x.w;
     }
     const int key = stage * kBwIT + (e >> 5) % kBwIT, d = (e & 31) * 4;

@@ -9,6 +9,8 @@ returns before a launch).
   of a sequence's routed pairs over its blocks, sum ceil(count / 256) fits.
 * The decode router refuses a k_bar cache with fewer than ceil(S / block_size) rows.
 * Split tiles ask for a workspace only where the library splits them.
+* The backward's parts of heavy key stages share one pool of slots, which holds the parts
+  of any documents and grows with their tokens, not with documents x longest document.
 """
 
 import ctypes
@@ -154,3 +156,66 @@ def test_split_tile_workspace():
     full = ctypes.c_int64(0)
     assert lib.dash_attn_prefill_workspace_size(1, 10, 2730, 2730, 8, 128, 64, full) == 0
     assert full.value >= _split_bytes(lib, 1, 10, 2730)
+
+
+def _bwd_bytes(lib, docs, K, bs, H=10):
+    n = ctypes.c_int64(0)
+    assert lib.dash_attn_prefill_backward_workspace_size(len(docs), H, max(docs), sum(docs), K, 128,
+                                                         bs, n) == 0
+    return n.value
+
+
+def _part_slots(rows, seqs, K, bs, per, X):
+    return 4 * per * (rows * K * bs + 64 * rows + 64 * seqs * bs) // (64 * bs * X)
+
+
+@pytest.mark.parametrize("docs", [[300] * 63 + [8192], [300] * 255 + [27300], [100] * 1000])
+def test_backward_workspace_follows_the_tokens(docs):
+    """At most the plan's own growth (chunk records and tile bases of every sequence are sized
+    for the longest) over the same tokens as documents of one length each, and over K = 1."""
+    lib = _lib_or_skip()
+    rows, K, bs, H = sum(docs), 16, 64, 10
+    full = _bwd_bytes(lib, docs, K, bs)
+    plan = ctypes.c_int64(0)
+    assert lib.dash_attn_prefill_workspace_size(len(docs), H, max(docs), rows, K, 128, bs, plan) == 0
+    # per pair, head: 256 B of dQ, 16 B of scales, 4 B of dbias (the forward's 136 B are part
+    # of `plan`); parts of at least 24 steps of 64 pairs: 64 KB for 4 / 24 of a step
+    pairs = rows * K + 256 * (rows // bs + len(docs) + 2)
+    parts = 4 * (pairs // 64 + rows // bs + len(docs)) // 24 * 65536 * H
+    assert full <= plan.value + pairs * H * 276 + parts + rows * H * 4 + (64 << 20)
+
+
+def test_backward_parts_fit_their_slots():
+    """Random documents and splits of their pairs over blocks: the parts of a sequence's stages
+    end before the next sequence's first slot, the last one's within the pool."""
+    rng = np.random.default_rng(11)
+    for _ in range(300):
+        bs = int(rng.choice([32, 64, 96, 128, 160, 192, 224, 256]))
+        K = int(rng.choice([1, 3, 12, 16, 64]))
+        lw = int(rng.choice([1, 64, 500]))
+        docs = [int(rng.choice([0, 1, 40, 300, 2000, 5000])) for _ in range(rng.integers(1, 7))]
+        nsub = (bs + 63) // 64
+        per = 1 if bs <= 64 else nsub if bs % 64 == 0 else nsub + 1
+        X = max(int(rng.integers(24, 129)), 2 * ((62 + lw) // 64 + 1))
+        row0 = 0
+        for b, n in enumerate(docs):
+            nblk = -(-n // bs)
+            pairs = n * K
+            counts = np.zeros(nblk, dtype=np.int64)
+            if nblk:                               # most pairs on a few blocks, or evenly
+                w = rng.random(nblk) ** rng.choice([0.0, 4.0, 30.0])
+                counts = np.minimum(rng.multinomial(pairs, w / w.sum()), n)
+            slots = 0
+            for j0 in range(0, nblk * bs, 64):
+                if j0 // bs * bs >= n:
+                    continue
+                t_end = min(j0 + 63 + lw - 1, n - 1)
+                steps = (t_end - j0) // 64 + 1 if t_end >= j0 else 0
+                first, last = j0 // bs, min(j0 + 63, n - 1) // bs
+                assert last <= first + 1
+                steps += sum(-(-int(c) // 64) for c in counts[first:max(first, last) + 1])
+                parts = max(1, -(-steps // X))
+                slots += parts if parts > 1 else 0
+            assert _part_slots(row0, b, K, bs, per, X) + slots <= \
+                _part_slots(row0 + n, b + 1, K, bs, per, X), (bs, K, lw, docs)
+            row0 += n
