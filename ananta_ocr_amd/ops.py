@@ -8,6 +8,7 @@ on the current HIP stream.  CPU tensors are rejected: the product has no CPU pat
 import ctypes
 import functools
 import math
+import threading
 
 import torch
 
@@ -646,11 +647,15 @@ def release_workspaces(device=None):
     synchronise first."""
     for k in [k for k in _WORKSPACES if device is None or k[1] == str(torch.device(device))]:
         del _WORKSPACES[k]
+    with _STEP_LOCK:
+        for k in [k for k in _STEP_WORKSPACES if device is None or k[0] == torch.device(device)]:
+            del _STEP_WORKSPACES[k]
 
 
 def cached_workspace_bytes():
     """Total bytes of the cached workspaces."""
-    return sum(b.numel() for b in _WORKSPACES.values())
+    with _STEP_LOCK:
+        return sum(b.numel() for c in (_WORKSPACES, _STEP_WORKSPACES) for b in c.values())
 
 
 def attn_prefill(q, k, v, idx, bias, valid, block_size, local_window, scale,
@@ -1260,8 +1265,9 @@ def decode_step_fused(q, k, v, idx_q, idx_k, head_cls, kbar_cache, block_size, l
         _lib.check(st_, "dash_decode_step_noalloc")
         return _step_result(out, lse, idx, bias, valid, z, squeeze, return_lse, return_scores)
     ws_bytes = _step_workspace_size(B, H, D, int(block_size), lw)
+    stream = _stream()
     if workspace is None:
-        ws = _step_workspace(ws_bytes, dev)
+        ws = _step_workspace(ws_bytes, dev, B, stream)
     else:
         ws = workspace
         if ws.numel() * ws.element_size() < ws_bytes:
@@ -1278,7 +1284,7 @@ def decode_step_fused(q, k, v, idx_q, idx_k, head_cls, kbar_cache, block_size, l
         out.data_ptr(), int(out_dtype == torch.bfloat16), H * D, D,
         _ptr(lse), 0 if lse is None else lse.stride(0), 1,
         B, H, D, int(block_size), lw, float(scale), ws.data_ptr(), ws.numel() * ws.element_size(),
-        _stream())
+        stream)
     if st_ != 0:
         _lib.check(st_, "dash_decode_step")
     if bare:
@@ -1294,24 +1300,52 @@ def _step_workspace_size(B, H, D, block_size, lw):
     return nbytes.value
 
 
+# Cached workspaces of decode steps, oldest first, at most as many as the limit.
 _STEP_WORKSPACES = {}
+STEP_WORKSPACE_LIMIT = 32
+_STEP_LOCK = threading.Lock()
 
 
-def _step_workspace(nbytes, device):
-    """The decode step's cached workspace on `device`: zeroed when it is allocated (the
-    routing words at its end must start at zero; every step leaves them zero), and
-    always passed whole, so those words stay in one place.  Calls that share it are
-    ordered on the current stream."""
-    k = device
+def _step_workspace(nbytes, device, B, stream):
+    """The decode step's workspace on `device` for `stream` (the current one) and this thread:
+    the two launches of a step hand each other partials and routing words in it, so steps on
+    other streams, or that another thread issues between the two, must not share it.  Zeroed
+    when it is allocated (the routing words at its end must start at zero; every step leaves
+    them zero), and always passed whole, so those words stay in one place.  Dropped ones
+    return to torch's allocator in the order of their stream.
+
+    A step recorded into a graph takes a buffer of the graph's own, whose words each replay
+    clears first (by a fill kernel): replays are ordered with nothing outside the graph.
+    Pass `workspace` (decode_step_workspace) to a recorded step to save that launch."""
+    if torch._C._cuda_isCurrentStreamCapturing():
+        buf = torch.empty((nbytes + 255) // 256 * 256, dtype=torch.uint8, device=device)
+        buf[buf.numel() - B * _STEP_WORD_BYTES:].zero_()
+        return buf
+    k = (device, stream, threading.get_ident())
     buf = _STEP_WORKSPACES.get(k)
-    if buf is None or buf.numel() * 4 < nbytes:
-        if buf is not None:
-            del _STEP_WORKSPACES[k]
-            del buf
-        buf = torch.zeros(((int(nbytes * 1.25) + 4095) // 4096) * 1024, dtype=torch.float32,
-                          device=device)
-        _STEP_WORKSPACES[k] = buf
+    if buf is None or buf.numel() < nbytes:
+        with _STEP_LOCK:
+            _STEP_WORKSPACES.pop(k, None)
+            buf = None                       # freed before its larger one is allocated
+            buf = torch.zeros(_step_alloc(nbytes * 1.25), dtype=torch.uint8, device=device)
+            _STEP_WORKSPACES[k] = buf
+            while len(_STEP_WORKSPACES) > STEP_WORKSPACE_LIMIT:
+                del _STEP_WORKSPACES[next(iter(_STEP_WORKSPACES))]
     return buf
+
+
+_STEP_WORD_BYTES = 256                       # routing words of a sequence
+
+
+def _step_alloc(nbytes):
+    return (int(nbytes) + 4095) // 4096 * 4096
+
+
+def decode_step_workspace(B, H, D, block_size, local_window, device):
+    """A zero-filled buffer for decode_step_fused's `workspace` (and pipeline.decode_step's)
+    for steps of up to B sequences that follow each other on one stream."""
+    n = _step_workspace_size(B, H, D, int(block_size), int(local_window))
+    return torch.zeros(_step_alloc(n), dtype=torch.uint8, device=device)
 
 
 def _step_result(out, lse, idx, bias, valid, z, squeeze, return_lse, return_scores):

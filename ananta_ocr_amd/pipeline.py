@@ -190,7 +190,7 @@ def init_decode_state(idx_k, head_cls, block_size, nblk_cap, seq_lens=None, bloc
 def decode_step(state, q, k, v, idx_q, idx_k, head_cls, block_size, local_blocks, idx_scale,
                 floor, sigma, K, topm, scale=None, seq_lens=None, block_table=None,
                 page_size=None, out_dtype=torch.float32, nsplit=None, block_cand=None,
-                return_routing=False, fused=None, return_scores=False, bounds=None):
+                return_routing=False, fused=None, return_scores=False, bounds=None, workspace=None):
     """One decode step for the query at the last cached token of each sequence.
     The newest token is already in k/v and idx_k; its block's summary is refreshed
     inside the fused decode router.  fused (default: whenever nsplit is not given and
@@ -199,7 +199,8 @@ def decode_step(state, q, k, v, idx_q, idx_k, head_cls, block_size, local_blocks
     (with return_routing) also returns the block scores [B, nblk_cap] of the router.
     state: a DecodeState (k_bar per sequence) or a KBarPageCache (k_bar per page, read
     through block_table; page_size must equal block_size).  bounds [B, 2]
-    (pages.win_bounds_decode of the candidate rows): only those blocks are scored."""
+    (pages.win_bounds_decode of the candidate rows): only those blocks are scored.
+    workspace: the fused step's buffer (ops.decode_step_workspace) instead of a cached one."""
     kbx = {}
     if state.paged:
         if block_table is None or page_size != block_size:
@@ -220,7 +221,7 @@ def decode_step(state, q, k, v, idx_q, idx_k, head_cls, block_size, local_blocks
             q, k, v, idx_q, idx_k, head_cls, state.kbar, block_size, local_blocks, idx_scale,
             floor, sigma, K, topm, scale, seq_lens=seq_lens, block_table=block_table,
             page_size=page_size, cand=block_cand, width=width, out_dtype=out_dtype,
-            return_scores=return_routing, return_routing=return_routing, **kbx)
+            return_scores=return_routing, return_routing=return_routing, workspace=workspace, **kbx)
         if not return_routing:
             return res
         out, (idx, bias, valid), z = res
@@ -248,14 +249,19 @@ class DecodeGraph:
     tensor ops between them) are recorded once; ``replay()`` relaunches them all
     with one host call, which is what a serving loop does for every token.  The
     inputs are the captured tensors themselves: write the new query (and the new
-    cache rows) into them in place before each replay.  Outputs live in buffers
-    owned by the graph and are overwritten by the next replay.
+    cache rows) into them in place before each replay.  Outputs and the step's
+    workspace live in buffers owned by the graph; the next replay overwrites them.
     """
 
     def __init__(self, state, q, k, v, idx_q, idx_k, head_cls, block_size, local_blocks,
                  idx_scale, floor, sigma, K, topm, scale=None, warmup=2, **kw):
         args = (state, q, k, v, idx_q, idx_k, head_cls, block_size, local_blocks, idx_scale,
                 floor, sigma, K, topm, scale)
+        if local_blocks > 0:
+            kw.setdefault("workspace", ops.decode_step_workspace(
+                q.shape[0], q.shape[1], q.shape[-1], block_size, local_blocks * block_size,
+                q.device))
+        self.workspace = kw.get("workspace")
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side):

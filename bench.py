@@ -371,12 +371,16 @@ def bench_paged_decode(cfg, steps, warmup):
         kv_bytes += a
         other += b
 
+    q0 = layers[0][0]["q"]
+    ws = ops.decode_step_workspace(q0.shape[0], q0.shape[1], q0.shape[-1], cfg.bs, lb * cfg.bs,
+                                   q0.device)
+
     def step(i=0):
         for d, st in layers:
             pipeline.decode_step(st, d["q"], d["k"], d["v"], d["idx_q"], d["idx_k"], hc, cfg.bs,
                                  lb, W.IDX_SCALE, W.FLOOR, W.SIGMA, cfg.cap, cfg.cap, scale,
                                  seq_lens=d["seq_lens"], block_table=d["block_table"],
-                                 page_size=cfg.bs)
+                                 page_size=cfg.bs, workspace=ws)
 
     t_step_eager = time_steps(step, steps, warmup)
     side = torch.cuda.Stream()
