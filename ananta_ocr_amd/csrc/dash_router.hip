@@ -2353,7 +2353,10 @@ extern "C" int dash_decode_step(
 // ---------------------------------------------------------------------------
 namespace dash {
 constexpr int64_t kStepScratchBytes = 64ll << 20;
-static __device__ __align__(256) float scratch[kStepScratchBytes / sizeof(float)];
+// Past the partials' bytes, the routing words of the largest step that has any (a grid of one
+// round, with a router on each CU), so that no step's partials reach another's words.
+constexpr int64_t kStepScratchWords = kDsCUs * kDcMaxK * 2 * 8;
+static __device__ __align__(256) float scratch[(kStepScratchBytes + kStepScratchWords) / sizeof(float)];
 constexpr int kMaxScratchDevices = 64;
 static std::atomic<float*> g_scratch_ptr[kMaxScratchDevices];
 static std::mutex g_scratch_mu;
@@ -2415,7 +2418,7 @@ extern "C" int dash_decode_step_noalloc(
                           K, topm, Kout, idx, bias, valid, z, z_stride, q, q_sb, q_sh, k, k_sb,
                           k_sh, k_st, k_sp, v, v_sb, v_sh, v_st, v_sp, out, out_bf16, o_sb, o_sh,
                           lse, lse_sb, lse_sh, B, H, D, block_size, local_window, scale, ptr,
-                          kStepScratchBytes, stream);
+                          kStepScratchBytes + kStepScratchWords, stream);
 }
 
 // ---------------------------------------------------------------------------

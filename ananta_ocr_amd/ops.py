@@ -1323,6 +1323,7 @@ def _step_workspace(nbytes, device, B, stream):
         return buf
     k = (device, stream, threading.get_ident())
     buf = _STEP_WORKSPACES.get(k)
+    nbytes += _STEP_WORDS                    # no step's partials reach the words of another
     if buf is None or buf.numel() < nbytes:
         with _STEP_LOCK:
             _STEP_WORKSPACES.pop(k, None)
@@ -1335,6 +1336,9 @@ def _step_workspace(nbytes, device, B, stream):
 
 
 _STEP_WORD_BYTES = 256                       # routing words of a sequence
+# The words of the largest step that has any: one whose grid is a single round of the 256 CUs,
+# a router on each.
+_STEP_WORDS = 256 * _STEP_WORD_BYTES
 
 
 def _step_alloc(nbytes):
@@ -1344,7 +1348,7 @@ def _step_alloc(nbytes):
 def decode_step_workspace(B, H, D, block_size, local_window, device):
     """A zero-filled buffer for decode_step_fused's `workspace` (and pipeline.decode_step's)
     for steps of up to B sequences that follow each other on one stream."""
-    n = _step_workspace_size(B, H, D, int(block_size), int(local_window))
+    n = _step_workspace_size(B, H, D, int(block_size), int(local_window)) + _STEP_WORDS
     return torch.zeros(_step_alloc(n), dtype=torch.uint8, device=device)
 
 

@@ -52,6 +52,21 @@ def test_the_cache_is_bounded_and_given_back(host):
     assert not ops._STEP_WORKSPACES and ops.cached_workspace_bytes() == 0
 
 
+def test_partials_of_one_step_end_below_the_words_of_another(host):
+    """A step of few sequences and many heads after one of more sequences: its partials, which
+    fill its own size but for its own words, end below the words of any step (256 bytes for
+    each of up to 255 sequences, at the buffer's end)."""
+    words = 255 * 256
+    ops._step_workspace(200000, torch.device("cpu"), 8, 0)
+    size = next(iter(ops._STEP_WORKSPACES.values())).numel()
+    for nbytes in range(size - 80000, size + 3000, 1000):
+        buf = ops._step_workspace(nbytes, torch.device("cpu"), 1, 0)
+        assert nbytes - 256 <= buf.numel() // 256 * 256 - words
+        buf = ops.decode_step_workspace(2, 300, 128, 64, nbytes // 500, "cpu")
+        assert buf.numel() // 256 * 256 - words >= ops._step_workspace_size(
+            2, 300, 128, 64, nbytes // 500) - 512
+
+
 def test_a_recorded_step_has_its_own_buffer(host):
     a = _get()
     host["capturing"] = True
