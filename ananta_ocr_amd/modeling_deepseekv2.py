@@ -31,7 +31,7 @@ import torch
 from . import ops, page_rope, pages
 from .dash_attention import DashAttention, apply_rotary, checkpoint_sparse_config
 
-_DASH_FORWARD_TRITON = DashAttention._forward_triton
+_DASH_FORWARDS = {n: getattr(DashAttention, n) for n in ("_forward_triton", "_forward_dense")}
 
 _INFER = {"on": False}
 
@@ -218,7 +218,8 @@ def _infer_prefill_attend(self, router, hidden_states, q, k, v, idx_pe, pos_ids,
     the reference does, and the decode state (index-key buffer and block summaries) in
     ``past_kv._dash_decode[layer_idx]``.  Attention goes through
     ``router._forward_triton`` and, where that returns None, ``router._forward_dense``,
-    as in the reference."""
+    as in the reference; bf16 without a mask goes to ``_forward_dense`` at once, unless
+    the router has a ``_forward_triton`` of its own."""
     B, H, S, D = q.shape
     nblk = (S + router.block_size - 1) // router.block_size
     p = router._infer_params
@@ -258,14 +259,20 @@ def _infer_prefill_attend(self, router, hidden_states, q, k, v, idx_pe, pos_ids,
     # host synchronisation in the middle of the prefill (with the launches that prepare it
     # 40 us of GPU work; 296 -> 222 us a layer of 2,730 tokens).  Routers with their own
     # _forward_triton, and types that the entry point refuses, still go through it.
-    own = getattr(type(router), "_forward_triton", None) is not _DASH_FORWARD_TRITON \
-        or "_forward_triton" in vars(router)
+    # Methods of a router's own get the ids in 64 bits, as _infer_route_select gives them.
     if router.use_triton and q.is_cuda and attn_mask is None \
-            and (own or q.dtype != torch.bfloat16):
+            and (_own(router, "_forward_triton") or q.dtype != torch.bfloat16):
         out = router._forward_triton(q, k, v, topi.long(), bias, valid, S, nblk, pos_ids)
         if out is not None:
             return out
+    if _own(router, "_forward_dense"):
+        topi = topi.long()
     return router._forward_dense(q, k, v, topi, bias, valid, S, nblk, attn_mask)
+
+
+def _own(router, name):
+    """Whether router's method `name` is not the package's."""
+    return name in vars(router) or getattr(type(router), name, None) is not _DASH_FORWARDS[name]
 
 
 # ----------------------------------------------------------------------------- decode
