@@ -19,8 +19,10 @@
 // Precision is that of the decode kernels: fp32 scores, weights, sums and partials.  A
 // weight enters the bf16 matrix product as three bf16 parts (24 significand bits), so it
 // is not rounded.  A row's result does not depend on the rows it shares a tile or chunk
-// with: window items start at multiples of 64 keys, masked keys add exact zeros, a pair's
-// partial involves its own block only, and the partials are added in slot order.
+// with: window items start at multiples of 64 keys, a pair's partial involves its own block
+// only, and the partials are added in slot order.  Masked keys add exact zeros where V is
+// finite; the window kernel gives a V value that is not to the rows that see its key, and a
+// routed block's reach the rows that name the block, as in the row-by-row kernels.
 #pragma once
 
 namespace dash {
@@ -98,15 +100,41 @@ __device__ __forceinline__ void ext_fetch(bf16* sX, const bf16* xb, const int32_
   }
 }
 
+// V values that are not finite would reach every row of an item through its products with
+// masked weights.  In a stage, just landed, each wavefront clears them in the rows it loaded
+// and returns the mask of the keys that hold any (its bit 4 u + i: row 16 u + 4 wv + i).
+__device__ __forceinline__ uint32_t ext_clear_rows(bf16* sX, int wv, int lane) {
+  uint32_t keys = 0;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    uint4* p = (uint4*)(sX + (4 * u + wv) * 4 * 128) + lane;
+    uint4 x = *p;
+    bool bad = false;
+    auto fix = [&](uint32_t& w) {
+      if ((w & 0x7f80u) == 0x7f80u) { w &= 0xffff0000u; bad = true; }
+      if ((w & 0x7f800000u) == 0x7f800000u) { w &= 0xffffu; bad = true; }
+    };
+    fix(x.x); fix(x.y); fix(x.z); fix(x.w);
+    if (bad) *p = x;
+    const uint64_t m = __ballot(bad);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) keys |= ((m >> (16 * i)) & 0xffffu) ? 1u << (4 * u + i) : 0u;
+  }
+  return keys;
+}
+
 // Bound by the matrix cores' chain per item (16 products of S^T, 48 of the three-part
 // P V) against the softmax's VALU work of the same 64 keys; K and V of the next item are
-// fetched meanwhile, two work-groups per CU.
+// fetched meanwhile, two work-groups per CU.  Where a work-group's result is not finite it
+// walks its band again, an item at a time, with V's finite values in the products, and adds
+// the others to the rows that see them.
 __global__ __launch_bounds__(256, 2) void extend_window_kernel(ExtendArgs a) {
   constexpr int D = 128;
   __shared__ __attribute__((aligned(16))) bf16 sK0[64 * D];
   __shared__ __attribute__((aligned(16))) bf16 sK1[64 * D];
   __shared__ __attribute__((aligned(16))) bf16 sV0[64 * D];
   __shared__ __attribute__((aligned(16))) bf16 sV1[64 * D];
+  __shared__ uint32_t sBad[4];             // keys of an item with values that are not finite
   const PrefillArgs& p = a.p;
   const int lid = xcd_logical_id(blockIdx.x, gridDim.x);
   const int g = lid % p.ntv, h = lid / p.ntv;
@@ -134,30 +162,26 @@ __global__ __launch_bounds__(256, 2) void extend_window_kernel(ExtendArgs a) {
   const int n_items = qlast >= 0 ? qlast / 64 - j_first / 64 + 1 : 0;
 
   floatx16 acc_o[D / 32];
+  float m_run, l_run;
+  auto reset = [&] {
+    m_run = -INFINITY;
+    l_run = 0.f;
 #pragma unroll
-  for (int dt = 0; dt < D / 32; ++dt)
+    for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc_o[dt][r] = 0.f;
-  float m_run = -INFINITY, l_run = 0.f;
+      for (int r = 0; r < 16; ++r) acc_o[dt][r] = 0.f;
+  };
   const int32_t* tr = a.table + (int64_t)b * a.table_stride;
   const bf16* kb = p.k + (int64_t)h * p.k_sh;
   const bf16* vb = p.v + (int64_t)h * p.v_sh;
   const uint32_t kl0 = k_lane_off(n, hl), vl0 = v_lane_off(lane);
   const float csc = p.scale_log2e;
 
-  auto step = [&](int it, auto par) {
+  // the item of keys j0 .. j0 + 63 in stage pair P
+  auto item = [&](int j0, auto par) __attribute__((always_inline)) {
     constexpr int P = decltype(par)::value;
     bf16* const sKc = P == 0 ? sK0 : sK1;
     bf16* const sVc = P == 0 ? sV0 : sV1;
-    bf16* const sKn = P == 0 ? sK1 : sK0;
-    bf16* const sVn = P == 0 ? sV1 : sV0;
-    const int j0 = j_first + it * 64;
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();                       // item it landed; every wavefront left it - 1
-    if (it + 1 < n_items) {
-      ext_fetch<0>(sKn, kb, tr, a.k_sp, p.k_st, p.bs, j0 + 64, klen, wv, lane);
-      ext_fetch<1>(sVn, vb, tr, a.v_sp, p.v_st, p.bs, j0 + 64, klen, wv, lane);
-    }
     if (!__any(qvalid && q_lo <= j0 + 63 && qp >= j0)) return;
     uint32_t kl = kl0, vl = vl0;
     asm volatile("" : "+v"(kl), "+v"(vl));
@@ -208,6 +232,20 @@ __global__ __launch_bounds__(256, 2) void extend_window_kernel(ExtendArgs a) {
         ext_pv(sVc, vl, 32 * hf + 16 * j, ph, pm, pl, acc_o);
       }
   };
+  auto step = [&](int it, auto par) __attribute__((always_inline)) {
+    constexpr int P = decltype(par)::value;
+    bf16* const sKn = P == 0 ? sK1 : sK0;
+    bf16* const sVn = P == 0 ? sV1 : sV0;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();                       // item it landed; every wavefront left it - 1
+    const int j0 = j_first + it * 64;
+    if (it + 1 < n_items) {
+      ext_fetch<0>(sKn, kb, tr, a.k_sp, p.k_st, p.bs, j0 + 64, klen, wv, lane);
+      ext_fetch<1>(sVn, vb, tr, a.v_sp, p.v_st, p.bs, j0 + 64, klen, wv, lane);
+    }
+    item(j0, par);
+  };
+  reset();
   if (n_items > 0) {
     ext_fetch<0>(sK0, kb, tr, a.k_sp, p.k_st, p.bs, j_first, klen, wv, lane);
     ext_fetch<1>(sV0, vb, tr, a.v_sp, p.v_st, p.bs, j_first, klen, wv, lane);
@@ -215,6 +253,44 @@ __global__ __launch_bounds__(256, 2) void extend_window_kernel(ExtendArgs a) {
   for (int it = 0; it < n_items; it += 2) {
     step(it, std::integral_constant<int, 0>{});
     if (it + 1 < n_items) step(it + 1, std::integral_constant<int, 1>{});
+  }
+  float z = 0.f;                           // NaN where a value is not finite
+#pragma unroll
+  for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) z = fmaf(acc_o[dt][r], 0.f, z);
+  if (__syncthreads_or(z != 0.f)) {
+    reset();
+    for (int it = 0; it < n_items; ++it) {
+      const int j0 = j_first + it * 64;
+      __syncthreads();                     // every wavefront left the stages
+      ext_fetch<0>(sK0, kb, tr, a.k_sp, p.k_st, p.bs, j0, klen, wv, lane);
+      ext_fetch<1>(sV0, vb, tr, a.v_sp, p.v_st, p.bs, j0, klen, wv, lane);
+      __builtin_amdgcn_s_waitcnt(0);
+      const uint32_t bad = ext_clear_rows(sV0, wv, lane);
+      if (lane == 0) sBad[wv] = bad;
+      __syncthreads();
+      item(j0, std::integral_constant<int, 0>{});
+      for (int w = 0; w < 4; ++w)
+        for (uint32_t todo = sBad[w]; todo; todo &= todo - 1) {
+          const int i = __builtin_ctz(todo), key = j0 + 16 * (i >> 2) + 4 * w + (i & 3);
+          if (key >= klen) continue;       // a repeated row
+          const bool sees = key >= q_lo && key <= qp;
+          const int blk = key / p.bs;
+          const bf16* vr = vb + (int64_t)tr[blk] * a.v_sp + (int64_t)(key - blk * p.bs) * p.v_st + 4 * hl;
+#pragma unroll
+          for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const bf16x4 x = *(const bf16x4*)(vr + 32 * dt + 8 * q);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const float f = (float)x[e];
+                if (sees && !(fabsf(f) <= 3.402823466e38f)) acc_o[dt][4 * q + e] += f;
+              }
+            }
+        }
+    }
   }
   const float l_tot = xor32_sum(l_run);
   if (qvalid) {

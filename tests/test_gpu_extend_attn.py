@@ -103,6 +103,38 @@ def test_extend_attention_matches_rows_and_exact(ctxs, news, H, bs, lw, K):
     assert torch.equal(half, got.bfloat16())
 
 
+@pytest.mark.parametrize("bs", [32, 64])
+def test_values_that_are_not_finite_stay_with_their_rows(bs):
+    """A V element that is not finite reaches the rows whose window holds its key and the rows
+    routed to its block, in its head and dim, and no others, which keep their bits."""
+    ctxs, news, H, lw, K = [300, 40], [200, 130], 2, 96, 4
+    q, k, v, idx, bias, valid, lens, table, cu = _make(ctxs, news, H, bs, K, 5, lw)
+    scale = 0.1
+    d = [torch.tensor(lens, device=DEV), torch.tensor(ctxs, device=DEV), cu.to(DEV), max(news),
+         table.to(DEV), bs, lw, scale]
+
+    def run(v):
+        return ops.attn_extend(*[x.to(DEV) for x in (q, k, v, idx, bias, valid)], *d).cpu()
+    clean = run(v)
+    assert clean.isfinite().all()
+    # request, key, head, dim: an old key, a key of the chunk (later than half of its rows, on
+    # a 64-key item's edge and within one), the last key
+    bad = [(0, 250, 0, 3, math.nan), (0, 383, 1, 77, math.inf), (0, 384, 0, 127, -math.inf),
+           (0, 405, 1, 0, math.inf), (1, 20, 1, 64, math.nan), (1, 169, 0, 9, math.nan)]
+    w = v.clone()
+    hit = torch.zeros(clean.shape, dtype=torch.bool)
+    for b, key, h, dim, x in bad:
+        w[table[b, key // bs], key % bs, h, dim] = x
+        for r in range(int(cu[b]), int(cu[b + 1])):
+            qp = ctxs[b] + r - int(cu[b])
+            routed = any(valid[r, s] and idx[r, s] == key // bs and key // bs * bs < qp - lw + 1
+                         for s in range(K))
+            hit[r, h, dim] |= qp - lw < key <= qp or routed
+    got = run(w)
+    assert torch.equal(~got.isfinite(), hit)
+    assert torch.equal(got[~hit], clean[~hit])
+
+
 def test_extend_attention_rows_do_not_depend_on_each_other():
     """Rows in another batch (other tiles, chunks and requests beside them), and q, k and v
     with other strides: the same bits."""
