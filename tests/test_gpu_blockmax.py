@@ -33,6 +33,18 @@ def _magnitude(q, k, bs, nblk):
     return torch.nn.functional.pad(m, (0, nblk * bs - k.shape[1])).view(*m.shape[:2], nblk, bs).amax(-1)
 
 
+def _bounds(q, k, pos, bs, nblk, lw):
+    """[B, C, nblk] least and largest block score of fp32 dot products in any order."""
+    s, e = q @ k.transpose(1, 2), DOT * (q.abs() @ k.abs().transpose(1, 2))
+    hidden = torch.arange(k.shape[1], device=q.device) > pos[..., None] - lw
+    out = []
+    for x in (s - e, s + e):
+        x = x.clamp(-1e4, 1e4).masked_fill(hidden, -1e9)
+        x = torch.nn.functional.pad(x, (0, nblk * bs - k.shape[1]), value=-1e9)
+        out.append(x.view(*x.shape[:2], nblk, bs).amax(-1))
+    return out
+
+
 @pytest.mark.parametrize("B,S,bs,lb", [(1, 1, 32, 1), (2, 31, 32, 1), (1, 333, 32, 4),
                                        (2, 700, 64, 2), (1, 385, 96, 1), (1, 641, 128, 1),
                                        (1, 4200, 32, 4), (1, 5000, 64, 1)])
@@ -45,8 +57,8 @@ def test_training_scores_and_gradients(B, S, bs, lb):
         ik[:, 40:44] = ik[:, 40:41]                 # equal keys within one block
         ik[:, 70] = 0.0
         iq[:, S - 1] *= 2.0e4                       # scores beyond the clamp
-        iq[0, S - 2] = 1.0e19                       # beyond the bf16 parts' range
-        ik[0, 100] *= 1.0e19
+        # beyond the bf16 parts' range (2^60 = 1.15e18); their products' sums stay in range
+        iq[0, S - 2], ik[0, 100] = 2.0e18, 2.0e18 * ik[0, 100]
     pos = torch.arange(S).expand(B, S).clone()
     if B > 1:
         pos[1] = torch.cat([torch.arange(S // 2), torch.arange(S - S // 2)])
@@ -56,8 +68,11 @@ def test_training_scores_and_gradients(B, S, bs, lb):
     z = r._block_scores_train(a, b, pos, nblk)
     c, d = iq.double().requires_grad_(), ik.double().requires_grad_()
     ref = r._block_scores_train(c, d, pos, nblk)    # 64-bit inputs: the tensor ops
-    tol = DOT * _magnitude(iq.double(), ik.double(), bs, nblk)
-    assert torch.all((z.double() - ref).abs() <= tol.clamp(max=1e30) + 1e-30)
+    # a masked block is exactly that; else the score lies between the largest of the visible
+    # keys' clamped lower bounds and that of their upper bounds
+    assert torch.equal(z == -1e9, ref == -1e9)
+    least, most = _bounds(iq.double(), ik.double(), pos, bs, nblk, lb * bs)
+    assert torch.all((z.double() >= least) & (z.double() <= most))
     # a gradient on a few entries of each row, the masked ones included
     dz = torch.randn(z.shape, generator=g).to(DEV)
     dz = torch.where(torch.rand(z.shape, generator=g).to(DEV) < 0.3, dz, torch.zeros_like(dz))
