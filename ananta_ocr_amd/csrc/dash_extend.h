@@ -80,6 +80,41 @@ __device__ __forceinline__ void ext_pv(const bf16* sVs, uint32_t vl, int kbase, 
     acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vop[dt], ph, acc_o[dt], 0, 0, 0);
 }
 
+// acc_o[dt] += V^T P^T over the 64 keys of a swizzled V stage, P in three parts.  The item's
+// products sum from zero, smallest parts first, before they meet the row's total: 12 roundings
+// at the item's size and one at the total's, instead of 12 at the total's.
+__device__ __forceinline__ void ext_pv_item(const bf16* sVs, uint32_t vl, const bf16x8 (&ph)[4],
+                                            const bf16x8 (&pm)[4], const bf16x8 (&pl)[4],
+                                            floatx16 (&acc_o)[4]) {
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt) {
+    bf16x8 vop[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const char* p = (const char*)sVs + ks * 16 * 256 + (vl ^ (uint32_t)(dt << 6));
+      const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_short4*)(__attribute__((address_space(3))) void*)p);
+      const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_short4*)(__attribute__((address_space(3))) void*)(p + 2048));
+      const bf16x4 l4 = __builtin_bit_cast(bf16x4, lo);
+      const bf16x4 h4 = __builtin_bit_cast(bf16x4, hi);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { vop[ks][e] = l4[e]; vop[ks][e + 4] = h4[e]; }
+    }
+    floatx16 t;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) t[r] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vop[ks], pl[ks], t, 0, 0, 0);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vop[ks], pm[ks], t, 0, 0, 0);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vop[ks], ph[ks], t, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc_o[dt][r] += t[r];
+  }
+}
+
 // Direct loads of keys j0 .. j0+63 (j0 a multiple of 32, j0 < klen) of one head into a
 // swizzled stage by 4 wavefronts: row 16 u + 4 wv + lane / 16.  Rows past the last key
 // repeat it, so that no unused row of the cache is read; the 16 rows of a group lie in one
@@ -217,20 +252,18 @@ __global__ __launch_bounds__(256, 2) void extend_window_kernel(ExtendArgs a) {
       m_run = up ? mloc : m_run;
     }
     const float off = m_run == -INFINITY ? 0.f : -m_run;
+    bf16x8 ph[4], pm[4], pl[4];
+    float l_item = 0.f;
 #pragma unroll
-    for (int hf = 0; hf < 2; ++hf)
+    for (int ks = 0; ks < 4; ++ks) {
+      float x[8];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        float x[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          x[e] = fast_exp2(fmaf(s[hf][8 * j + e], csc, off));
-          l_run += x[e];
-        }
-        bf16x8 ph, pm, pl;
-        ext_split3(x, ph, pm, pl);
-        ext_pv(sVc, vl, 32 * hf + 16 * j, ph, pm, pl, acc_o);
-      }
+      for (int e = 0; e < 8; ++e) x[e] = fast_exp2(fmaf(s[ks >> 1][8 * (ks & 1) + e], csc, off));
+      l_item += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+      ext_split3(x, ph[ks], pm[ks], pl[ks]);
+    }
+    l_run += l_item;
+    ext_pv_item(sVc, vl, ph, pm, pl, acc_o);
   };
   auto step = [&](int it, auto par) __attribute__((always_inline)) {
     constexpr int P = decltype(par)::value;

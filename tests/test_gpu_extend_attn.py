@@ -97,7 +97,8 @@ def test_extend_attention_matches_rows_and_exact(ctxs, news, H, bs, lw, K):
     ref = _exact(*data, ctxs, bs, lw, scale, rows)
     err = (got[rows].cpu().double() - ref).norm() / ref.norm()
     old_err = (old[rows].cpu().double() - ref).norm() / ref.norm()
-    assert err <= 2 * old_err + 2e-7, (err, old_err)
+    # no further from 64 bits than the row-by-row kernels (0.78 to 0.94 of their error here)
+    assert err <= 1.05 * old_err, (err, old_err)
     half = ops.attn_extend(*d, ln, ctx, cu.to(DEV), max(news), table.to(DEV), bs, lw, scale,
                            out_dtype=torch.bfloat16)
     assert torch.equal(half, got.bfloat16())
