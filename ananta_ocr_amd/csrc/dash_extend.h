@@ -87,41 +87,31 @@ __device__ __forceinline__ void ext_pv_item(const bf16* sVs, uint32_t vl, const 
                                             const bf16x8 (&pm)[4], const bf16x8 (&pl)[4],
                                             floatx16 (&acc_o)[4]) {
 #pragma unroll
-  for (int d0 = 0; d0 < 4; d0 += 2) {      // two chains at a time
-    bf16x8 vop[2][4];
+  for (int dt = 0; dt < 4; ++dt) {
+    bf16x8 vop[4];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
+    for (int ks = 0; ks < 4; ++ks) {
+      const char* p = (const char*)sVs + ks * 16 * 256 + (vl ^ (uint32_t)(dt << 6));
+      const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_short4*)(__attribute__((address_space(3))) void*)p);
+      const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_short4*)(__attribute__((address_space(3))) void*)(p + 2048));
+      const bf16x4 l4 = __builtin_bit_cast(bf16x4, lo);
+      const bf16x4 h4 = __builtin_bit_cast(bf16x4, hi);
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const char* p = (const char*)sVs + ks * 16 * 256 + (vl ^ (uint32_t)((d0 + u) << 6));
-        const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (lds_short4*)(__attribute__((address_space(3))) void*)p);
-        const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (lds_short4*)(__attribute__((address_space(3))) void*)(p + 2048));
-        const bf16x4 l4 = __builtin_bit_cast(bf16x4, lo);
-        const bf16x4 h4 = __builtin_bit_cast(bf16x4, hi);
+      for (int e = 0; e < 4; ++e) { vop[ks][e] = l4[e]; vop[ks][e + 4] = h4[e]; }
+    }
+    floatx16 t;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) { vop[u][ks][e] = l4[e]; vop[u][ks][e + 4] = h4[e]; }
-      }
-    floatx16 t[2];
+    for (int r = 0; r < 16; ++r) t[r] = 0.f;
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int ks = 0; ks < 4; ++ks) t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vop[ks], pl[ks], t, 0, 0, 0);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) t[u][r] = 0.f;
-    auto add = [&](const bf16x8 (&x)[4]) {
+    for (int ks = 0; ks < 4; ++ks) t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vop[ks], pm[ks], t, 0, 0, 0);
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks)
+    for (int ks = 0; ks < 4; ++ks) t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vop[ks], ph[ks], t, 0, 0, 0);
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-          t[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vop[u][ks], x[ks], t[u], 0, 0, 0);
-    };
-    add(pl);
-    add(pm);
-    add(ph);
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc_o[d0 + u][r] += t[u][r];
+    for (int r = 0; r < 16; ++r) acc_o[dt][r] += t[r];
   }
 }
 
