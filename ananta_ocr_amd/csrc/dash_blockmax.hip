@@ -4,11 +4,12 @@
 //   ls(t) = max(pos(t) - LW + 1, 0)      (dash_attention.py:801-835,
 //                                         sparse_gather_triton.py:395-428)
 //
-//   blockmax_f32_kernel     inference: 128 query rows x up to 1,024 keys per work-group by
+//   blockmax_f32_kernel     inference: 128 query rows x up to 128 keys per work-group by
 //                           fp32 matrix products, the bits of the row-by-row kernel
 //   blockmax_split_kernel   training: fp32 keys -> three bf16 parts per key, in the LDS
 //                           image of a 32-key tile
-//   blockmax_mfma_kernel    training: the same tiles by products of the bf16 parts
+//   blockmax_mfma_kernel    training: 128 query rows x up to 1,024 keys per work-group by
+//                           products of the bf16 parts
 //   blockmax_bwd_q_kernel   dq of every row from the winning keys, and the bit mask of
 //                           the (row, block) pairs with a gradient
 //   blockmax_bwd_k_kernel   dk of every key from that mask; blockmax_bwd_sum_kernel adds
@@ -39,6 +40,7 @@ constexpr int kBmTileBytes = 3 * kBmPlane * 2;    // 24 KB
 constexpr int kBmRows = 128;                      // query rows per work-group
 constexpr int kBmMaxChunk = 1024;                 // keys per work-group, at most
 constexpr int kBmMaxBlocks = kBmMaxChunk / 32;    // blocks per work-group, at most
+constexpr int kBmF32Chunk = 128;                  // keys per work-group of the fp32 kernel, at most
 constexpr int kBmSlow = 255;                      // no single winning key
 constexpr int kBmRange = 4096;                    // query rows per dk work-group
 constexpr float kBmWide = 1.152921504606847e18f;  // 2^60
@@ -78,13 +80,13 @@ __device__ __forceinline__ void bm_split3(float x, __bf16& h, __bf16& m, __bf16&
 // S^T = K Q^T gives lane l the scores of query l % 32, so the maximum over a block's keys is
 // per lane, with one exchange between the wave's halves.  Key tiles stream through two 16 KB
 // stages by direct loads.  Bound by the matrix products, 4,096 cycles per wavefront and tile
-// (1,536 with bf16 parts, which need the keys split first): 2,730 rows and keys in blocks of
-// 32 26.0 us (row by row 93.9, bf16 parts 25.5), 2,730 rows of 27,300 keys 218 (754), one row
-// of 2,730 keys 11.0 (16.0).
+// (1,536 with bf16 parts, which need the keys split first), at half their rate.  In blocks of
+// 32, 2,730 rows and keys take 26.9 us (row by row 93.9, bf16 parts 24.2), 8,301 133.3 (bf16 parts
+// 85.6), 2,730 rows of 27,300 keys 206.9 (753.7, 138.9), one row of 2,730 keys 7.3 (16.0, 15.8).
 __global__ __launch_bounds__(256, 3) void blockmax_f32_kernel(BlockMaxArgs a) {
   __shared__ __attribute__((aligned(16))) float s0[kBmTile * 128];
   __shared__ __attribute__((aligned(16))) float s1[kBmTile * 128];
-  __shared__ float sOut[4][32][kBmMaxBlocks + 1];
+  __shared__ float sOut[4][32][kBmF32Chunk / 32 + 1];
   __shared__ int sHi[4];
   const int b = blockIdx.z, r0 = blockIdx.x * kBmRows;
   const int tid = threadIdx.x, lane = wave_lane(), wv = tid / kWave;
@@ -692,16 +694,18 @@ extern "C" int dash_block_max_fused(const float* q, int64_t q_sb, int64_t q_st, 
   a.nblk = nblk; a.mode = mode; a.ntiles = nt;
   a.out = out; a.o_sb = o_sb; a.o_sc = o_sc; a.arg = arg;
   hipStream_t st = (hipStream_t)stream;
-  // keys per work-group: 1,024 (the rows are read once per work-group, scores leave in
-  // 64-byte or longer pieces), halved while the grid holds too few work-groups
-  auto blocks_per_group = [&](int least, int64_t groups) {
-    int keys = kBmMaxChunk;
+  // keys per work-group: as many as let the rows' reads serve many keys, halved while the
+  // grid holds too few work-groups
+  auto blocks_per_group = [&](int most, int least, int64_t groups) {
+    int keys = most;
     while (keys > least && (int64_t)rt * B * ((nt * kBmTile + keys - 1) / keys) < groups) keys /= 2;
     return std::max(1, keys / block_size);
   };
   if (mode != 2 && !arg) {
     if (B == 0 || C == 0 || nblk == 0) return kOk;
-    const int bpc = blocks_per_group(64, 1024);
+    // blocks of 32: 1,000 rows and keys 10.1 us with 32 keys (21.2 with 128), 2,730 26.9 with 64
+    // (30.6 with 32, 31.8 with 128), 8,301 133.3 with 128 (140.7 with 64, 189.8 with 1,024)
+    const int bpc = blocks_per_group(kBmF32Chunk, 32, 512);
     a.chunk_tiles = bpc * tpb;
     blockmax_f32_kernel<<<dim3(rt, (nblk + bpc - 1) / bpc, B), 256, 0, st>>>(a);
     return bm_status();
@@ -715,7 +719,8 @@ extern "C" int dash_block_max_fused(const float* q, int64_t q_sb, int64_t q_st, 
   char* const planes = (char*)ws;
   int32_t* const wide = (int32_t*)(planes + (int64_t)B * nt * kBmTileBytes);
   blockmax_split_kernel<<<dim3(nt, B), 256, 0, st>>>(k, k_sb, k_st, Sk, nt, planes, wide);
-  const int bpc = blocks_per_group(256, 512);
+  // scores leave in 64-byte or longer pieces with 1,024 keys
+  const int bpc = blocks_per_group(kBmMaxChunk, 256, 512);
   a.planes = planes; a.wide = wide; a.chunk_tiles = bpc * tpb;
   const dim3 grid(rt, (nblk + bpc - 1) / bpc, B);
   if (arg)

@@ -179,8 +179,9 @@ def block_max_score(q, k, pos, seg, block_size, num_key_blocks, local_window, mo
 
 
 # Fewest query rows per sequence for the matrix-core block-max kernel, which gives the bits of
-# the row-by-row kernel: any number.  389 to 27,300 keys, batches of 1 and 8, blocks of 32 and
-# 64: 1 row 10.5 to 56 us against 16 to 144 row by row, 2,730 rows of 2,730 keys 26 against 94.
+# the row-by-row kernel: any number.  Blocks of 32: 1 row of 2,730 keys 7.3 us against 16.0 row
+# by row, 8 sequences with 1 row of 27,300 keys 57.7 against 144, 2,730 rows and keys 26.9
+# against 93.9.
 BLOCK_MAX_FUSED_ROWS = 1
 
 
