@@ -5,13 +5,13 @@ and the ``forward`` signature of the reference module (dash_attention.py:703-107
 so that the DeepSeek-V2 decoder can use it unchanged.
 
 ``forward`` is the reference's training forward (dash_attention.py:1008-1071):
-stage-0 block scores from the router's index projections (indexer block-max or
-head_cls summaries, in PyTorch so that autograd reaches the projections, norms and
-head_cls), then the training router in ``libdash_hip.so`` (full-width 1.5-entmax
-prior, top-k of the masked prior with k from the global schedule, centred
-log-prior bias; dash_train_route with its backward), then the fused block-sparse
-attention in ``libdash_hip.so`` with gradients to q, k, v and the bias
-(dash_attn_prefill and dash_attn_prefill_backward).
+stage-0 block scores from the router's index projections (projections, norms and
+indexer block-max scores in ``libdash_hip.so`` with their gradients where the inputs
+and modules allow it; otherwise, and for head_cls summaries, by tensor ops), then the
+training router in ``libdash_hip.so`` (full-width 1.5-entmax prior, top-k of the
+masked prior with k from the global schedule, centred log-prior bias; dash_train_route
+with its backward), then the fused block-sparse attention in ``libdash_hip.so`` with
+gradients to q, k, v and the bias (dash_attn_prefill and dash_attn_prefill_backward).
 
 The inference form (modeling_deepseekv2.py:309-333: top-M by score, entmax over
 the M, first K) is ``route``; ``_infer_params`` holds {idx_scale, floor, sigma, K,

@@ -883,8 +883,8 @@ PROBE_KERNELS = {
     "decode": ["decode_route_window_kernel", "decode_routed_kernel", "decode_step_merge_kernel"],
     "front": ["router_front_kernel"],
     "train": ["bwd_delta_kernel", "prefill_clear_kernel", "prefill_plan_kernel",
-              "prefill_scan_kernel", "prefill_scatter_kernel", "bwd_kv_kernel", "bwd_q_kernel",
-              "bwd_dbias_kernel"],
+              "prefill_scan_kernel", "prefill_scatter_kernel", "bwd_items_kernel",
+              "bwd_kv_kernel", "bwd_sum_kernel", "bwd_q_kernel", "bwd_dbias_kernel"],
 }
 
 
