@@ -623,20 +623,42 @@ DENSE_THRESHOLD = 48   # of the 128 queries of a tile; below it a routed block g
 SMALL_TILES = 256
 SMALL_BLOCKS = 64
 
+# Cached workspaces by kind, device and stream, oldest first, at most WORKSPACE_LIMIT of a kind
+# and device.
+# _WORKSPACE_LOCK is held from taking one to the end of the call that enqueues its launches,
+# so that another thread's launches on the stream do not fall between them.
 _WORKSPACES = {}
+WORKSPACE_LIMIT = 8
+_WORKSPACE_LOCK = threading.RLock()
+
+
+def _device_stream(device):
+    """(current stream of `device` as a raw handle, whether it is being recorded into a graph);
+    (0, False) for host memory."""
+    if device.type != "cuda":
+        return 0, False
+    index = torch.cuda.current_device() if device.index is None else device.index
+    return torch._C._cuda_getCurrentRawStream(index), torch._C._cuda_isCurrentStreamCapturing()
 
 
 def cached_workspace(key, nbytes, device):
-    """A cached device buffer of at least `nbytes` (contents undefined; the kernels
-    clear what they count in).  Calls that share it are ordered on the current stream."""
-    k = (key, str(device))
-    buf = _WORKSPACES.get(k)
-    if buf is None or buf.numel() < nbytes:
-        if buf is not None:
-            del _WORKSPACES[k]
-            del buf
-        buf = torch.empty(int(nbytes * 1.1) + 4096, dtype=torch.uint8, device=device)
-        _WORKSPACES[k] = buf
+    """A cached device buffer of at least `nbytes` for the current stream (contents undefined;
+    the kernels clear what they count in).  Calls on one stream share it in order; each stream
+    has its own, and a call recorded into a graph takes memory of the graph's."""
+    stream, capturing = _device_stream(torch.device(device))
+    if capturing:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    k = (key, str(device), stream)
+    with _WORKSPACE_LOCK:
+        buf = _WORKSPACES.get(k)
+        if buf is None or buf.numel() < nbytes:
+            if buf is not None:
+                del _WORKSPACES[k]
+                del buf
+            buf = torch.empty(int(nbytes * 1.1) + 4096, dtype=torch.uint8, device=device)
+            _WORKSPACES[k] = buf
+            for o in [o for o in _WORKSPACES if o[:2] == k[:2]][:-WORKSPACE_LIMIT]:
+                del _WORKSPACES[o]
     return buf
 
 
@@ -646,8 +668,9 @@ def release_workspaces(device=None):
     again.  Safe between calls on one stream (torch hands freed memory out again in
     stream order); with work that used a workspace still running on another stream,
     synchronise first."""
-    for k in [k for k in _WORKSPACES if device is None or k[1] == str(torch.device(device))]:
-        del _WORKSPACES[k]
+    with _WORKSPACE_LOCK:
+        for k in [k for k in _WORKSPACES if device is None or k[1] == str(torch.device(device))]:
+            del _WORKSPACES[k]
     with _STEP_LOCK:
         for k in [k for k in _STEP_WORKSPACES if device is None or k[0] == torch.device(device)]:
             del _STEP_WORKSPACES[k]
@@ -655,7 +678,7 @@ def release_workspaces(device=None):
 
 def cached_workspace_bytes():
     """Total bytes of the cached workspaces."""
-    with _STEP_LOCK:
+    with _WORKSPACE_LOCK, _STEP_LOCK:
         return sum(b.numel() for c in (_WORKSPACES, _STEP_WORKSPACES) for b in c.values())
 
 
@@ -712,19 +735,20 @@ def attn_prefill(q, k, v, idx, bias, valid, block_size, local_window, scale,
     elif rows > 0 and split_tiles:
         # every routed block with its tile: the partials of split tiles (small grids)
         _lib.check(lib.dash_attn_prefill_split_workspace_size(nb, H, Smax, D, nbytes), "workspace")
-    if nbytes.value > 0:
-        ws = cached_workspace("prefill", nbytes.value, q.device)
-        ws_n = ws.numel()
     km = _i32(kmin)
-    st_ = lib.dash_attn_prefill(
-        _ptr(q), q.stride(0), q.stride(1), q.stride(2),
-        _ptr(k), k.stride(0), k.stride(1), k.stride(2),
-        _ptr(v), v.stride(0), v.stride(1), v.stride(2),
-        _ptr(o), o.stride(0), o.stride(1), o.stride(2),
-        _ptr(lse), H, 1,
-        _ptr(idx_c), _ptr(valid_c), _ptr(bias_c), K, _ptr(cu), _ptr(km),
-        nb, H, Smax, D, int(block_size), int(local_window), float(scale),
-        thr, rows, _ptr(ws), ws_n, _stream())
+    with _WORKSPACE_LOCK:
+        if nbytes.value > 0:
+            ws = cached_workspace("prefill", nbytes.value, q.device)
+            ws_n = ws.numel()
+        st_ = lib.dash_attn_prefill(
+            _ptr(q), q.stride(0), q.stride(1), q.stride(2),
+            _ptr(k), k.stride(0), k.stride(1), k.stride(2),
+            _ptr(v), v.stride(0), v.stride(1), v.stride(2),
+            _ptr(o), o.stride(0), o.stride(1), o.stride(2),
+            _ptr(lse), H, 1,
+            _ptr(idx_c), _ptr(valid_c), _ptr(bias_c), K, _ptr(cu), _ptr(km),
+            nb, H, Smax, D, int(block_size), int(local_window), float(scale),
+            thr, rows, _ptr(ws), ws_n, _stream())
     _lib.check(st_, "dash_attn_prefill")
     return (o, lse) if return_lse else o
 
@@ -763,21 +787,22 @@ def attn_prefill_backward(q, k, v, o, lse, dout, idx, bias, valid, block_size, l
     _lib.check(lib.dash_attn_prefill_backward_workspace_size(nb, H, Smax, rows, K, D,
                                                              int(block_size), nbytes),
                "workspace")
-    ws = cached_workspace("prefill_bwd", nbytes.value, q.device)
     km = _i32(kmin)
-    st_ = lib.dash_attn_prefill_backward(
-        _ptr(q), q.stride(0), q.stride(1), q.stride(2),
-        _ptr(k), k.stride(0), k.stride(1), k.stride(2),
-        _ptr(v), v.stride(0), v.stride(1), v.stride(2),
-        _ptr(o), o.stride(0), o.stride(1), o.stride(2),
-        _ptr(dout), dout.stride(0), dout.stride(1), dout.stride(2),
-        _ptr(lse), H, 1,
-        _ptr(idx_c), _ptr(valid_c), _ptr(bias_c), K, _ptr(cu), _ptr(km),
-        nb, H, Smax, D, int(block_size), int(local_window), float(scale),
-        _ptr(dq), dq.stride(0), dq.stride(1), dq.stride(2),
-        _ptr(dk), dk.stride(0), dk.stride(1), dk.stride(2),
-        _ptr(dv), dv.stride(0), dv.stride(1), dv.stride(2),
-        _ptr(dbias), rows, _ptr(ws), ws.numel(), _stream())
+    with _WORKSPACE_LOCK:
+        ws = cached_workspace("prefill_bwd", nbytes.value, q.device)
+        st_ = lib.dash_attn_prefill_backward(
+            _ptr(q), q.stride(0), q.stride(1), q.stride(2),
+            _ptr(k), k.stride(0), k.stride(1), k.stride(2),
+            _ptr(v), v.stride(0), v.stride(1), v.stride(2),
+            _ptr(o), o.stride(0), o.stride(1), o.stride(2),
+            _ptr(dout), dout.stride(0), dout.stride(1), dout.stride(2),
+            _ptr(lse), H, 1,
+            _ptr(idx_c), _ptr(valid_c), _ptr(bias_c), K, _ptr(cu), _ptr(km),
+            nb, H, Smax, D, int(block_size), int(local_window), float(scale),
+            _ptr(dq), dq.stride(0), dq.stride(1), dq.stride(2),
+            _ptr(dk), dk.stride(0), dk.stride(1), dk.stride(2),
+            _ptr(dv), dv.stride(0), dv.stride(1), dv.stride(2),
+            _ptr(dbias), rows, _ptr(ws), ws.numel(), _stream())
     _lib.check(st_, "dash_attn_prefill_backward")
     return dq, dk, dv, dbias
 
@@ -1304,7 +1329,7 @@ def _step_workspace_size(B, H, D, block_size, lw):
 # Cached workspaces of decode steps, oldest first, at most as many as the limit.
 _STEP_WORKSPACES = {}
 STEP_WORKSPACE_LIMIT = 32
-_STEP_LOCK = threading.Lock()
+_STEP_LOCK = threading.RLock()
 
 
 def _step_workspace(nbytes, device, B, stream):
