@@ -626,7 +626,9 @@ SMALL_BLOCKS = 64
 # Cached workspaces by kind, device and stream, oldest first, at most WORKSPACE_LIMIT of a kind
 # and device.
 # _WORKSPACE_LOCK is held from taking one to the end of the call that enqueues its launches,
-# so that another thread's launches on the stream do not fall between them.
+# so that another thread's launches on the stream do not fall between them.  It also guards the
+# decode steps' cache: with two locks a finalizer that gives workspaces back, run inside one
+# thread's allocation, could wait for another thread's.
 _WORKSPACES = {}
 WORKSPACE_LIMIT = 8
 _WORKSPACE_LOCK = threading.RLock()
@@ -671,14 +673,13 @@ def release_workspaces(device=None):
     with _WORKSPACE_LOCK:
         for k in [k for k in _WORKSPACES if device is None or k[1] == str(torch.device(device))]:
             del _WORKSPACES[k]
-    with _STEP_LOCK:
         for k in [k for k in _STEP_WORKSPACES if device is None or k[0] == torch.device(device)]:
             del _STEP_WORKSPACES[k]
 
 
 def cached_workspace_bytes():
     """Total bytes of the cached workspaces."""
-    with _WORKSPACE_LOCK, _STEP_LOCK:
+    with _WORKSPACE_LOCK:
         return sum(b.numel() for c in (_WORKSPACES, _STEP_WORKSPACES) for b in c.values())
 
 
@@ -1329,7 +1330,6 @@ def _step_workspace_size(B, H, D, block_size, lw):
 # Cached workspaces of decode steps, oldest first, at most as many as the limit.
 _STEP_WORKSPACES = {}
 STEP_WORKSPACE_LIMIT = 32
-_STEP_LOCK = threading.RLock()
 
 
 def _step_workspace(nbytes, device, B, stream):
@@ -1351,7 +1351,7 @@ def _step_workspace(nbytes, device, B, stream):
     buf = _STEP_WORKSPACES.get(k)
     nbytes += _STEP_WORDS                    # no step's partials reach the words of another
     if buf is None or buf.numel() < nbytes:
-        with _STEP_LOCK:
+        with _WORKSPACE_LOCK:
             _STEP_WORKSPACES.pop(k, None)
             buf = None                       # freed before its larger one is allocated
             buf = torch.zeros(_step_alloc(nbytes * 1.25), dtype=torch.uint8, device=device)
